@@ -47,9 +47,9 @@ CLOCK_HZ = 2.4e9
 # library bracket plan + trace + finalize of every round (the trace kernel is
 # > 97% of a round in the kernel traces under profiles/)
 DOMINANT = "hase_queue_trace_kernel"
-# its instantiation on meshes staged in LDS as compact records (<refill lanes,
-# problem table, LDS record kind: 1 compact, 2 indexed>)
-STAGED_TRACE = "hase_queue_trace_kernel<false, false, 1u>"
+# its instantiation on meshes whose edge records fit in LDS (<refill lanes,
+# problem table, edge record kind: 4 with coordinates, 5 indexed, 6 twins>)
+STAGED_TRACE = "hase_queue_trace_kernel<false, false, 4u>"
 # algorithmic cost of one prism step of the walk (rays and importance walks)
 BYTES_PER_STEP = 56
 FLOPS_PER_STEP = 40
@@ -219,7 +219,7 @@ def kernel_table(stats, queue=True):
         trace: {"launches": launches, "avg_ms": trace_ms / max(launches, 1), "ms": trace_ms,
                 "prism_steps": ray_steps, "rays": rays,
                 "flops_per_launch": (ray_steps * FLOPS_PER_STEP + rays * FLOPS_PER_RAY) / max(launches, 1)},
-        "hase_importance_kernel": {"launches": imp_launches, "avg_ms": imp_ms / max(imp_launches, 1), "ms": imp_ms,
+        "hase_column_map_kernel": {"launches": imp_launches, "avg_ms": imp_ms / max(imp_launches, 1), "ms": imp_ms,
                                    "prism_steps": imp_steps,
                                    "flops_per_launch": imp_steps * FLOPS_PER_STEP / max(imp_launches, 1)},
     }
@@ -602,7 +602,7 @@ def combined_bench(args):
 def traffic_pass(w, args):
     """Kernels for the FETCH_SIZE / WRITE_SIZE counter runs: the learned
     evaluation (its hase_trace_kernel launches are the bench line's), a plain
-    evaluation of the first level's samples (hase_importance_kernel), and a
+    evaluation of the first level's samples (hase_column_map_kernel), and a
     1 GiB device fill + device-to-device copy (the runtime's fillBuffer and
     copyBuffer kernels) whose known byte counts calibrate the counters."""
     from haseongpu_amd import proposal as prop

@@ -36,12 +36,17 @@ struct hase_context {
     std::vector<double> sigma_a, sigma_e;
     hase_compute_t comp{};
     hase::DevBuf<uint4> rec, lds_rec;
-    hase::DevBuf<uint4> cmp_rec;       // compact records beside indexed ones (kind kLdsIndexed)
-    uint32_t lds_kind = 0;             // format of lds_rec: 0 (none), kLdsCompact, kLdsIndexed or kCompactGlobal
-    bool lds_staged() const { return lds_kind == hase::kLdsCompact || lds_kind == hase::kLdsIndexed; }
+    hase::DevBuf<uint4> edges;         // edge records in global memory
+    uint32_t lds_kind = 0;             // edge format of lds_rec: 0 (none), kLdsEdges, kLdsIndexedEdges or kLdsTwins
+    bool lds_staged() const { return lds_kind != 0u; }
     hase::DevBuf<float2> pts;
     hase::DevBuf<float> beta, beta_col, bv, refl, c1, c2;
     hase::DevBuf<float> imp;
+    uint32_t path_cap = 32;            // triangles of an importance path that the map kernel stores
+    uint64_t path_tiles = 0;           // tiles of 64 paths that the storage holds
+    hase::DevBuf<uint2> path;          // triangles and exit sigmas of a sub-batch of paths
+    hase::DevBuf<uint32_t> path_head;  // a head per path of it
+    hase::DevBuf<uint32_t> path_over, path_count;   // longer paths of the resident samples, and how many
     hase::DevBuf<double> prefix, Q, s1, s2, bcells;
     hase::DevBuf<uint32_t> buckets;    // [batch * kPrefixBuckets] prefix buckets per resident sample
     hase::DevBuf<double2> partial;

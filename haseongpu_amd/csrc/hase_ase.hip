@@ -2,12 +2,12 @@
 // C ABI of include/hase_ase.h.
 //
 // Device pipeline per batch of sample points:
-//   1. hase_importance_kernel (one work-group per sample): walks from every
-//      prism centroid (and its mirror slices) to the sample point, forms the
-//      defensive-mixture proposal and writes its FP64 inclusive prefix.  This
-//      fuses the legacy importanceSamplingPropagation and
-//      importanceSamplingDistribution passes (retired; shells at
-//      include/kernels/importanceSampling.hpp:10-18).
+//   1. hase_column_map_kernel: walks from every prism centroid (and its
+//      mirror slices) to the sample point, along the xy path that a triangle
+//      column's levels and slices share; hase_prefix_kernel
+//      forms the defensive-mixture proposal and its FP64 inclusive prefix (the
+//      legacy importanceSamplingPropagation and importanceSamplingDistribution
+//      passes; retired, shells at include/kernels/importanceSampling.hpp:10-18).
 //   2. hase_trace_kernel (work-groups of one sample's ray chunk): maps each ray
 //      to its (slice, prism) by systematic sampling on the device prefix (the
 //      legacy host loop mapRaysToPrisms, shell include/kernels/mapRaysToTets.hpp),
@@ -34,6 +34,7 @@
 #include "../../include/hase_ase.h"
 #include "common.h"
 #include "context.h"
+#include "edge_records.h"
 #include "prism_walk.h"
 #include "importance_walk.h"
 #include "proposal.h"
@@ -206,160 +207,177 @@ struct ImportanceParams {
     const uint32_t* active;   // block -> slot (nullptr: block index is the slot)
     const uint32_t* sample_of;// slot -> sample (nullptr: sample_base + slot)
     int transfer;             // write the transfer factor gain * reflectance instead of the importance
-    uint32_t parts;           // work-groups per sample; > 1: importance only, hase_prefix_kernel follows
 };
 
-// kKind: the records the walks read from global memory: 0 the 48-byte
-// records, kCompactGlobal the 32-byte compact records.
-template <uint32_t kKind>
-__global__ void __launch_bounds__(kBlock) hase_importance_kernel(ImportanceParams p)
-{
-    const uint32_t row = blockIdx.x / p.parts, part = blockIdx.x % p.parts;
-    const uint32_t slot = p.active ? p.active[row] : row;
-    if (slot >= p.slots) return;
-    const MeshDev& m = p.m;
-    const uint32_t T = m.T, P = T * m.layers;
-    const size_t n = (size_t)p.R * P;
-    const uint32_t sample = p.sample_of ? p.sample_of[slot] : p.sample_base + slot;
-    SampleGeom sp = sample_point(p.pts, m.np, sample);
-    float* imp = p.imp + (size_t)slot * n;
-    double* pre = p.prefix + (size_t)slot * n;
-    const int tid = threadIdx.x, lane = tid & 63;
-    __shared__ double red[kBlock / 64 + 2];
-    __shared__ double buf[kScanLds];
+// The walked importance map.  A path is the xy segment from a triangle
+// column's centroid to a sample point: every level and reflection slice of
+// the column shares it.  Paths are handled in tiles of 64 neighbouring columns
+// of one sample, a sub-batch of tiles at a time:
+//   hase_column_path_kernel  walks the paths, one per lane (vertex and
+//                            neighbour fetches, side test, reciprocal), and
+//                            stores each one's triangles and exit sigmas;
+//   hase_column_map_kernel   replays a tile from LDS, one ray (slice, layer,
+//                            column) per lane, columns fastest: the lanes of a
+//                            wavefront follow neighbouring paths at one slope,
+//                            cross the same planes together, and their beta
+//                            reads (level-major, triangles in Hilbert order)
+//                            share cache lines.
+// Walked apart, the paths keep the whole chip's wavefronts busy; walked by the
+// replaying work-group (one wavefront walking, the others waiting) they took
+// half of its time.
+//
+// A path longer than its storage (path_cap triangles, from the mesh's extent
+// and density) is put on a list for hase_column_list_kernel, which walks its
+// column as column_entries does, level group by level group.
+constexpr uint32_t kTilePaths = 64;
+constexpr uint32_t kMapBlock = 512;
+constexpr uint32_t kPathEntries = 4096;   // 32 KiB of LDS: 4 work-groups of 512 threads per CU
 
-    double local = 0.0;
-    unsigned long long walks = 0, steps = 0;
-    const ColumnItems ci(T, m.layers, p.R);
-    const uint32_t items = ci.per_sample();
-    // this work-group's share of the sample's column walks
-    const uint32_t it0 = (uint32_t)((uint64_t)items * part / p.parts);
-    const uint32_t it1 = (uint32_t)((uint64_t)items * (part + 1u) / p.parts);
-    for (uint32_t it = it0 + tid; it < it1; it += kBlock) {
-        uint32_t t0, k;
-        int lv0, nlev;
-        ci.decode(it, t0, k, lv0, nlev);
-        float v[kLevelGroup];
-        if constexpr (kKind != 0u)
-            steps += column_entries(m, staged_fetch<kKind>(m.lds_rec, T), p.c1, p.c2, p.n_lambda, p.inv_lambda, t0, lv0,
-                                    nlev, k, sp.px, sp.py, sp.plane, p.transfer != 0, v);
-        else
-            steps += column_entries(m, GlobalTriangles{}, p.c1, p.c2, p.n_lambda, p.inv_lambda, t0, lv0, nlev, k, sp.px,
-                                    sp.py, sp.plane, p.transfer != 0, v);
-        walks += (unsigned long long)nlev;
-#pragma unroll
-        for (int g = 0; g < kLevelGroup; ++g) {
-            if (g < nlev) {
-                imp[(size_t)k * P + t0 + (uint32_t)(lv0 + g) * T] = v[g];
-                local += (double)v[g];
-            }
-        }
-    }
-    unsigned long long ws = wave_sum_u64(walks), ss = wave_sum_u64(steps);
-    if (lane == 0 && ws) {
-        atomicAdd(&p.counters[2], ws);
-        atomicAdd(&p.counters[3], ss);
-    }
-    if (p.transfer || p.parts > 1u) return;
-    mixture_prefix(local, (uint32_t)n, P, T, m.bv, p.eps, p.Bsum, p.R,
-                   [&](const EntryIndex&, uint32_t e) { return imp[e]; }, pre, p.Q + slot, red, buf,
-                   p.buckets ? p.buckets + (size_t)slot * kPrefixBuckets : nullptr);
+struct PathHead {
+    uint32_t steps;       // triangles stored (0: on the list, or no column); bit 31: reached its end
+    float clad, s;        // sum of dsigma over cladding triangles, sigma reached
+    float d2;             // squared xy length
+};
+
+struct PathParams {
+    ImportanceParams p;
+    uint2* path;          // [tiles of a sub-batch][rows][64] {4 * triangle, sigma bits}
+    PathHead* head;       // [tiles of a sub-batch][64]
+    uint32_t* over_count; // one word, zero before the launch
+    uint32_t* over;       // [slots * T] listed paths (slot * T + t0); null: the list kernel walks every path
+    uint32_t rows;        // entries of a path's storage, the end mark included
+    uint64_t tile0;       // tiles [tile0, tile0 + ntiles) of the batch's slots * ceil(T / 64)
+    uint32_t ntiles;
+    uint32_t inv_layers;  // ceil(2^32 / layers)
+};
+
+__device__ __forceinline__ SampleGeom path_sample(const ImportanceParams& p, uint32_t slot)
+{
+    return sample_point(p.pts, p.m.np, p.sample_of ? p.sample_of[slot] : p.sample_base + slot);
 }
 
-// Walked importance of whole batches for meshes of up to kLdsTriangles
-// triangles: one persistent 1024-thread work-group per CU copies the compact
-// triangle records into LDS once, then its wavefronts take 256 consecutive
-// column items of the batch at a time, round-robin over the grid (a batch's
-// items are numbered slot-major, so a wavefront's items are neighbouring
-// triangle columns of one sample and slice), and walk them in four rounds
-// of 64 sorted by estimated work.  Only the
-// importance values are written; hase_prefix_kernel forms each sample's
-// mixture prefix afterwards (not for transfer maps).
-constexpr int kStagedBlock = 1024;
-
-template <uint32_t kKind>
-__global__ void __launch_bounds__(kStagedBlock) hase_importance_staged_kernel(ImportanceParams p)
+__global__ void __launch_bounds__(kBlock) hase_column_path_kernel(PathParams q)
 {
-    __shared__ uint4 s_tri[kLdsStageWords];
+    const ImportanceParams& p = q.p;
     const MeshDev& m = p.m;
-    const uint32_t T = m.T, P = T * m.layers;
-    for (uint32_t i = threadIdx.x; i < m.lds_words; i += blockDim.x) s_tri[i] = m.lds_rec[i];
-    __syncthreads();
-    const auto fetch = staged_fetch<kKind>(s_tri, T);
-    const size_t n = (size_t)p.R * P;
-    const ColumnItems ci(T, m.layers, p.R);
-    const uint32_t per_slot = ci.per_sample();
-    const uint64_t total = (uint64_t)p.slots * per_slot;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t waves_per_block = blockDim.x / 64u;
-    const uint64_t wave = (uint64_t)blockIdx.x * waves_per_block + threadIdx.x / 64u;
-    const uint64_t stride = (uint64_t)gridDim.x * waves_per_block * 256u;
+    const uint32_t T = m.T, lane = threadIdx.x & 63u;
+    // the wavefront's tile, in scalar registers
+    const uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)));
+    if (at >= q.ntiles) return;
+    const uint32_t tiles = (T + kTilePaths - 1u) / kTilePaths;
+    const uint32_t slot = (uint32_t)((q.tile0 + at) / tiles);
+    const uint32_t t0 = (uint32_t)(q.tile0 + at - (uint64_t)slot * tiles) * kTilePaths + lane;
+    const SampleGeom sp = path_sample(p, slot);
+    uint2* out = q.path + (size_t)at * q.rows * kTilePaths + lane;
+    PathHead h{0u, 0.0f, 0.0f, 0.0f};
+    if (t0 < T) {
+        const ColumnPath path = column_path(m, GlobalEdges{}, t0, sp.px, sp.py,
+                                            [&](uint32_t step, uint32_t t, float sigma) {
+            if (step + 1u >= q.rows) return false;
+            out[(size_t)step * kTilePaths] = make_uint2(4u * t, __float_as_uint(sigma));
+            return true;
+        });
+        out[(size_t)path.steps * kTilePaths] = make_uint2(0u, kPathEnd);
+        h = PathHead{path.full ? 0u : path.steps | (path.ok ? 0x80000000u : 0u), path.clad, path.s, path.d2};
+        if (path.full) q.over[atomicAdd(q.over_count, 1u)] = slot * T + t0;
+    }
+    q.head[(size_t)at * kTilePaths + lane] = h;
+}
+
+__global__ void __launch_bounds__(kMapBlock, 8) hase_column_map_kernel(PathParams q)
+{
+    __shared__ uint2 s_path[kPathEntries + kTilePaths];   // [row][column]; one row past the last may be read
+    __shared__ PathHead s_head[kTilePaths];
+    const ImportanceParams& p = q.p;
+    const MeshDev& m = p.m;
+    const uint32_t T = m.T, layers = m.layers, P = T * layers, tid = threadIdx.x;
+    const uint32_t tiles = (T + kTilePaths - 1u) / kTilePaths;
+    // work-groups are dealt to the 8 XCDs round-robin: each XCD takes one
+    // contiguous eighth of the tiles, in order, so neighbouring ones share
+    // its L2
+    const uint32_t xcd = blockIdx.x & 7u;
+    const uint32_t g1 = (uint32_t)((uint64_t)q.ntiles * (xcd + 1u) >> 3);
     unsigned long long steps = 0;
-    // Items 256 at a time per wavefront, sorted by estimated work (the
-    // column's triangle crossings, from its centroid's xy distance to the
-    // sample at 1.2 sqrt(T / mesh area) per cm, times its levels, plus their
-    // plane crossings) and taken as four rounds of 64: lanes of a round walk
-    // columns of similar length, whose plane crossings fall on similar steps.
-    for (uint64_t base = wave * 256u; base < total; base += stride) {
-        // slot and item of the group's first item (wavefront-uniform); item
-        // base + li is li further on, in the same slot or the next ones
-        const uint64_t slot0 = base / per_slot;
-        const uint32_t it0 = (uint32_t)(base - slot0 * per_slot);
-        auto locate = [&](uint32_t li, uint32_t& slot, uint32_t& it) {
-            slot = (uint32_t)slot0;
-            it = it0 + li;
-            while (it >= per_slot) {
-                it -= per_slot;
-                ++slot;
+    for (uint32_t g = (uint32_t)((uint64_t)q.ntiles * xcd >> 3) + (blockIdx.x >> 3); g < g1; g += gridDim.x >> 3) {
+        const uint32_t slot = (uint32_t)((q.tile0 + g) / tiles);
+        const uint32_t t00 = (uint32_t)(q.tile0 + g - (uint64_t)slot * tiles) * kTilePaths;
+        const uint32_t cols = min(kTilePaths, T - t00);
+        const SampleGeom sp = path_sample(p, slot);
+        const uint2* paths = q.path + (size_t)g * q.rows * kTilePaths;
+        // columns that LDS holds at once, from the tile's longest path
+        const PathHead mine = q.head[g * kTilePaths + (tid & 63u)];
+        uint32_t rows = (mine.steps & 0x7FFFFFFFu) + 1u;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) rows = max(rows, (uint32_t)__shfl_xor((int)rows, off, 64));
+        rows = (uint32_t)__builtin_amdgcn_readfirstlane((int)rows);
+        uint32_t shift = 6u;
+        while (shift && (rows << shift) > kPathEntries) --shift;
+        const uint32_t hold = 1u << shift;
+        for (uint32_t c0 = 0; c0 < cols; c0 += hold) {
+            __syncthreads();   // the previous columns have been replayed
+            for (uint32_t i = tid; i < rows << shift; i += kMapBlock)
+                s_path[i] = paths[(i >> shift) * kTilePaths + c0 + (i & (hold - 1u))];
+            if (tid < kTilePaths) s_head[tid] = mine;
+            __syncthreads();
+            // (slice, layer, column) rays, columns fastest
+            for (uint32_t i = tid; i < (p.R * layers) << shift; i += kMapBlock) {
+                const uint32_t c = i & (hold - 1u), kl = i >> shift;
+                if (c0 + c >= cols) continue;
+                const uint32_t k = layers == 1u ? kl : __umulhi(kl, q.inv_layers), l = kl - k * layers;
+                const PathHead h = s_head[c0 + c];
+                if (h.steps == 0u) continue;
+                const uint32_t j = t00 + c0 + c + l * T;
+                const float bv = m.bv[j];
+                uint32_t visited = h.steps & 0x7FFFFFFFu;
+                float v = 0.0f;
+                if ((h.steps >> 31) && (bv > 0.0f || p.transfer)) {
+                    const uint32_t nr = (k + 1u) >> 1, first = k & 1u;
+                    const int end = image_plane(sp.plane, (int)layers, nr, first);
+                    PathRay w = path_ray_begin(m, (int)l, end);
+                    const uint32_t last = path_ray_replay(m, w, h.d2, nr, s_path + c, hold);
+                    visited += path_ray_planes(w, (int)l, end);
+                    v = path_ray_value(m, w, last, h.clad, h.s, h.d2, nr, first, p.c1, p.c2, p.n_lambda, p.inv_lambda,
+                                       bv, p.transfer != 0);
+                }
+                steps += visited;
+                p.imp[((size_t)slot * p.R + k) * P + j] = v;
             }
-            return slot < p.slots;
-        };
-        uint32_t key[4];
-#pragma unroll
-        for (uint32_t r = 0; r < 4u; ++r) {
-            const uint32_t li = r * 64u + lane;
-            key[r] = 0xFFFFFF00u | li;   // past the end: sorted last, skipped
-            uint32_t slot, it;
-            if (locate(li, slot, it)) {
-                const uint32_t sample = p.sample_of ? p.sample_of[slot] : p.sample_base + slot;
-                const SampleGeom sp = sample_point(p.pts, m.np, sample);
-                uint32_t t0, k;
-                int lv0, nlev;
-                ci.decode(it, t0, k, lv0, nlev);
-                const float2 a = fetch.vertex(m, t0, 0u), b = fetch.vertex(m, t0, 1u), c = fetch.vertex(m, t0, 2u);
-                const float dx = (a.x + b.x + c.x) * (1.0f / 3.0f) - sp.px, dy = (a.y + b.y + c.y) * (1.0f / 3.0f) - sp.py;
-                const float ze = (float)image_plane(sp.plane, (int)m.layers, (k + 1u) >> 1, k & 1u);
-                const float est = (float)nlev * (sqrtf(dx * dx + dy * dy) * m.steps_per_cm +
-                                                 fabsf((float)lv0 + 0.5f * (float)nlev - ze));
-                key[r] = ((uint32_t)fminf(est * 4.0f, 16777214.0f) << 8) | li;
-            }
-        }
-        wave_sort256(key, (int)lane);
-        uint32_t items4 = 0u;   // the four group indices, 8 bits each
-#pragma unroll
-        for (uint32_t r = 0; r < 4u; ++r) items4 |= (key[r] & 0xFFu) << (8u * r);
-#pragma unroll 1
-        for (uint32_t r = 0; r < 4u; ++r, items4 >>= 8) {
-            uint32_t slot, it;
-            if (!locate(items4 & 0xFFu, slot, it)) continue;
-            const uint32_t sample = p.sample_of ? p.sample_of[slot] : p.sample_base + slot;
-            const SampleGeom sp = sample_point(p.pts, m.np, sample);
-            uint32_t t0, k;
-            int lv0, nlev;
-            ci.decode(it, t0, k, lv0, nlev);
-            float v[kLevelGroup];
-            steps += column_entries(m, fetch, p.c1, p.c2, p.n_lambda, p.inv_lambda, t0, lv0, nlev, k, sp.px, sp.py,
-                                    sp.plane, p.transfer != 0, v);
-            float* imp = p.imp + (size_t)slot * n + (size_t)k * P + t0;
-#pragma unroll
-            for (int g = 0; g < kLevelGroup; ++g)
-                if (g < nlev) imp[(size_t)(lv0 + g) * T] = v[g];
         }
     }
-    // every entry of every slot is one level walk
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&p.counters[2], (unsigned long long)p.slots * n);
-    const unsigned long long ss = wave_sum_u64(steps);
-    if (lane == 0 && ss) atomicAdd(&p.counters[3], ss);
+    __shared__ unsigned long long red[kMapBlock / 64u];
+    block_count(steps, red, &p.counters[3]);
+}
+
+// Columns of the listed paths (every path without a list) by whole column
+// walks: one item per path, slice and level group.
+__global__ void __launch_bounds__(kBlock) hase_column_list_kernel(PathParams q)
+{
+    const ImportanceParams& p = q.p;
+    const MeshDev& m = p.m;
+    const uint32_t T = m.T, P = T * m.layers;
+    const ColumnItems ci(1u, m.layers, p.R);   // items of one column
+    const uint32_t per = ci.per_sample();
+    const uint64_t paths = q.over ? *q.over_count : (uint64_t)p.slots * T;
+    const uint64_t items = paths * per;
+    unsigned long long steps = 0;
+    for (uint64_t it = blockIdx.x * (uint64_t)kBlock + threadIdx.x; it < items; it += (uint64_t)gridDim.x * kBlock) {
+        const uint64_t a = it / per;
+        const uint64_t i = q.over ? q.over[a] : a;
+        const uint32_t slot = (uint32_t)(i / T), t0 = (uint32_t)(i - (uint64_t)slot * T);
+        const SampleGeom sp = path_sample(p, slot);
+        uint32_t unused, k;
+        int lv0, nlev;
+        ci.decode((uint32_t)(it - a * per), unused, k, lv0, nlev);
+        float v[kLevelGroup];
+        steps += column_entries(m, GlobalTriangles{}, p.c1, p.c2, p.n_lambda, p.inv_lambda, t0, lv0, nlev, k, sp.px,
+                                sp.py, sp.plane, p.transfer != 0, v);
+        float* imp = p.imp + ((size_t)slot * p.R + k) * P + t0;
+#pragma unroll
+        for (int g = 0; g < kLevelGroup; ++g)
+            if (g < nlev) imp[(size_t)(lv0 + g) * T] = v[g];
+    }
+    __shared__ unsigned long long red[kBlock / 64];
+    block_count(steps, red, &p.counters[3]);
 }
 
 // beta * V proposal shared by every sample (one work-group): the mixture with
@@ -375,7 +393,7 @@ __global__ void __launch_bounds__(kBlock) hase_beta_volume_prefix_kernel(Importa
                    p.prefix, p.Q, red, buf, p.buckets);
 }
 
-// Prefix of importance maps written by split work-groups (one per sample here).
+// Mixture prefix of the importance maps, one work-group per sample.
 __global__ void __launch_bounds__(kBlock) hase_prefix_kernel(ImportanceParams p)
 {
     const uint32_t slot = p.active ? p.active[blockIdx.x] : blockIdx.x;
@@ -950,61 +968,39 @@ std::unique_ptr<hase_context> create_context(const hase_mesh_t* mesh, const hase
         double area = 0.0;
         for (uint32_t td = 0; td < T; ++td) area += ctx->tri_area[td];
         ctx->steps_per_cm = 1.2 * std::sqrt((double)T / area);
+        // storage of an importance path: a straight line across a mesh of
+        // even density crosses up to ~1.6 sqrt(T / area) triangles per cm
+        double x0 = px[0], x1 = px[0], y0 = py[0], y1 = py[0], r2 = 0.0;
+        for (uint32_t i = 0; i < np; ++i) {
+            x0 = std::min(x0, px[i]); x1 = std::max(x1, px[i]);
+            y0 = std::min(y0, py[i]); y1 = std::max(y1, py[i]);
+        }
+        for (uint32_t i = 0; i < np; ++i) {
+            const double dx = px[i] - 0.5 * (x0 + x1), dy = py[i] - 0.5 * (y0 + y1);
+            r2 = std::max(r2, dx * dx + dy * dy);
+        }
+        const double most = 16.0 + 1.9 * std::sqrt((double)T / area) * 2.0 * std::sqrt(r2);
+        ctx->path_cap = (uint32_t)std::min(10000.0, std::max(32.0, std::ceil(most / 16.0) * 16.0));
     }
     ctx->rec.upload(rec.data(), rec.size(), ctx->stream);
     ctx->user2dev_dev.upload(ctx->user2dev.data(), T, ctx->stream);
-    const bool indexed_fits = T < (1u << 19) && np <= 0x10000u && (size_t)T + (np + 1u) / 2u <= hase::kLdsStageWords;
-    // compact records (corners + 21-bit neighbour fields + cladding bit) of
-    // every mesh below 2^19 triangles: staged in LDS up to kLdsTriangles,
-    // else read from global memory by the walks that do not stage
-    std::vector<uint4> crec;
-    if (T < (1u << 19)) {
-        crec.resize(2u * (size_t)T);
-        for (uint32_t td = 0; td < T; ++td) {
-            const uint4 a = rec[3u * td], b = rec[3u * td + 1u], c = rec[3u * td + 2u];
-            const uint32_t nwk[3] = {b.z, b.w, c.x};
-            uint64_t W = 0;
-            for (int k = 0; k < 3; ++k) {
-                const uint64_t f = nw_boundary(nwk[k]) ? 0x1FFFFFull
-                                                       : (uint64_t)(nw_next(nwk[k]) << 2 | nw_edge(nwk[k]));
-                W |= f << (21 * k);
-            }
-            W |= (uint64_t)(c.y >> 31) << 63;
-            crec[2u * td] = a;
-            crec[2u * td + 1u] = make_uint4(b.x, b.y, (uint32_t)W, (uint32_t)(W >> 32));
-        }
-    }
-    if (T <= hase::kLdsTriangles || (!indexed_fits && !crec.empty())) {
-        ctx->lds_rec.upload(crec.data(), crec.size(), ctx->stream);
-        ctx->lds_kind = T <= hase::kLdsTriangles ? hase::kLdsCompact : hase::kCompactGlobal;
-    } else if (indexed_fits) {
-        // indexed records (point indices + the compact records' neighbour
-        // word) followed by the vertex table; the compact records stay in
-        // global memory beside them
-        std::vector<uint4> lrec((size_t)T + (np + 1u) / 2u, make_uint4(0u, 0u, 0u, 0u));
-        for (uint32_t td = 0; td < T; ++td) {
-            const uint4 c = rec[3u * td + 2u], q = crec[2u * td + 1u];
-            const uint32_t clad = c.y >> 31;
-            lrec[td] = make_uint4((c.y & 0x7FFFFFFFu) | c.z << 16, c.w | clad << 31, q.z, q.w);
-        }
-        float2* vtx = reinterpret_cast<float2*>(lrec.data() + T);
-        for (uint32_t i = 0; i < np; ++i) vtx[i] = make_float2((float)px[i], (float)py[i]);
-        ctx->lds_rec.upload(lrec.data(), lrec.size(), ctx->stream);
-        ctx->lds_kind = hase::kLdsIndexed;
-        ctx->cmp_rec.upload(crec.data(), crec.size(), ctx->stream);
-    }
-    if (ctx->lds_staged()) {
-        // staged walks run one 1024-thread work-group per CU
-        ctx->tuning.stage_lds = 1u;
-        ctx->tuning.block_size = 1024u;
-        ctx->tuning.rays_per_item = 512u;
-    } else if (ctx->lds_kind == hase::kCompactGlobal) {
-        ctx->tuning.stage_lds = 1u;
-    }
-    ctx->centroid.upload(ctx->centroid_host.data(), T, ctx->stream);
     std::vector<float2>& pts = ctx->pts_host;
     pts.resize(np);
     for (uint32_t i = 0; i < np; ++i) pts[i] = make_float2((float)px[i], (float)py[i]);
+    {
+        const EdgeRecords er = edge_records(rec.data(), T, pts.data(), np);
+        ctx->edges.upload(er.global.data(), er.global.size(), ctx->stream);
+        if (er.kind) ctx->lds_rec.upload(er.staged.data(), er.staged.size(), ctx->stream);
+        ctx->lds_kind = er.kind;
+        HIP_CHECK(hipStreamSynchronize(ctx->stream));
+    }
+    ctx->tuning.stage_lds = 1u;
+    if (ctx->lds_staged()) {
+        // staged walks run one 1024-thread work-group per CU
+        ctx->tuning.block_size = 1024u;
+        ctx->tuning.rays_per_item = 512u;
+    }
+    ctx->centroid.upload(ctx->centroid_host.data(), T, ctx->stream);
     ctx->pts.upload(pts.data(), np, ctx->stream);
     if (mesh->reflectivities) {
         ctx->has_refl = true;
@@ -1035,7 +1031,7 @@ MeshDev mesh_view(const hase_context* ctx)
     m.rec = ctx->rec.p;
     m.lds_rec = ctx->lds_rec.p;
     m.lds_kind = ctx->lds_rec.p ? ctx->lds_kind : 0u;
-    m.cmp_rec = ctx->lds_kind == kLdsIndexed ? ctx->cmp_rec.p : (ctx->lds_rec.p ? ctx->lds_rec.p : nullptr);
+    m.edges = ctx->edges.p;
     m.lds_words = (uint32_t)ctx->lds_rec.n;
     m.beta = ctx->beta.p;
     m.beta_col = ctx->beta_col.p;
@@ -1046,6 +1042,8 @@ MeshDev mesh_view(const hase_context* ctx)
     m.T = ctx->T;
     m.layers = ctx->L - 1;
     m.np = ctx->np;
+    m.by_T = fast_div(m.T);
+    m.by_P = fast_div(m.T * m.layers);
     m.h = (float)ctx->h;
     m.clad_alpha = (float)ctx->clad_alpha;
     m.steps_per_cm = (float)ctx->steps_per_cm;
@@ -1066,6 +1064,45 @@ struct BatchTimers {
     std::vector<std::pair<hipEvent_t, hipEvent_t>> imp, trace, fin, inf, prop;
     double queue_ms = 0.0;
 };
+
+// Path storage of the walked importance map: at most kPathScratch bytes per
+// context (a sub-batch of the production disk is then ~100 samples, 22 million
+// rays, far more than fill the chip), less where the map is smaller, halved
+// while the device cannot give it; and the list of `paths` paths.  Returns the
+// tiles it holds, 0 where not even one fits.
+constexpr size_t kPathScratch = (size_t)512 << 20;
+
+uint64_t reserve_paths(hase_context* ctx, uint64_t tiles, size_t paths)
+{
+    const size_t rows = std::min(ctx->path_cap, kPathEntries - 1u) + 1u;
+    const size_t per = kTilePaths * (rows * sizeof(uint2) + sizeof(PathHead));
+    // allocation-free calls: an eighth of the scratch, reserved by their first call
+    const size_t budget = g_arena ? (ctx->path_tiles ? ctx->path_tiles * per : g_arena->remaining() / 8u) : kPathScratch;
+    uint64_t want = std::min<uint64_t>({tiles, std::max<size_t>(budget / per, g_arena ? 0u : 1u), 1u << 24});
+    try {
+        if (paths > ctx->path_over.n) {
+            if (g_arena && g_arena->remaining() < (paths + 64u) * sizeof(uint32_t)) return 0;
+            ctx->path_over.alloc(paths);
+        }
+        ctx->path_count.alloc(1);
+        while (want > ctx->path_tiles) {
+            try {
+                ctx->path.alloc(want * rows * kTilePaths);
+                ctx->path_head.alloc(want * kTilePaths * (sizeof(PathHead) / sizeof(uint32_t)));
+                ctx->path_tiles = want;
+            } catch (const HaseError& e) {
+                if (e.code != HASE_E_MEMORY || want == 1u) throw;
+                ctx->path_tiles = 0;
+                want /= 2u;
+            }
+        }
+    } catch (const HaseError& e) {
+        if (e.code != HASE_E_MEMORY) throw;
+        (void)hipGetLastError();
+        ctx->path_tiles = 0;
+    }
+    return ctx->path_tiles;
+}
 
 // Device buffers for batches of up to `want` resident samples; returns the
 // batch size.  Unless the caller fixed sample_batch, the importance prefix and
@@ -1097,10 +1134,15 @@ uint32_t reserve_batch(hase_context* ctx, uint32_t want, size_t budget = 0, bool
         // allocation-free call: as many slots as the scratch left after the
         // mesh holds (64 KiB kept for the per-call tables and alignment)
         const size_t tables_b = n_ent * 12u + kPrefixBuckets * 4u;
-        const size_t per_slot = (shared ? 0u : tables_b) + chunks * 20u + 256u +
-                                (learned ? (size_t)R * ctx->C * 4u : 0u);
-        size_t left = g_arena->remaining();
+        size_t per_slot = (shared ? 0u : tables_b) + chunks * 20u + 256u +
+                          (learned ? (size_t)R * ctx->C * 4u : 0u);
         const size_t keep = ((size_t)64 << 10) + (shared ? tables_b : 0u);
+        // importance paths and their list, where several slots fit beside
+        // them (the map's columns are walked level group by level group else)
+        if (!shared && ctx->path_tiles == 0 && g_arena->remaining() / 8u > per_slot + keep)
+            reserve_paths(ctx, (uint64_t)1 << 32, 0);
+        if (ctx->path_tiles) per_slot += ctx->T * sizeof(uint32_t);
+        size_t left = g_arena->remaining();
         left = left > keep ? left - keep : 0u;
         const size_t fit = std::min<size_t>(left / per_slot, 8192);
         if (fit == 0)
@@ -1162,49 +1204,39 @@ uint32_t reserve_batch(hase_context* ctx, uint32_t want, size_t budget = 0, bool
     return batch;
 }
 
-// Work-groups per sample for the walked importance map: enough to give a
-// small batch two work-groups per CU.
-uint32_t importance_parts(const hase_context* ctx, uint32_t slots)
-{
-    int cus = 0;
-    HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
-    const uint32_t want = 2u * (uint32_t)std::max(1, cus);
-    if (slots >= want) return 1u;
-    return std::min<uint32_t>(64u, (want + slots - 1u) / slots);
-}
-
 // Walked importance of `slots` samples (and, unless ip.transfer is set, their
-// mixture prefixes): the LDS-staged persistent kernel when the mesh's compact
-// records exist, else one work-group per sample (split into ip.parts for
-// small batches).  ip.parts is set here.
+// mixture prefixes).
 void launch_importance(hase_context* ctx, ImportanceParams& ip, uint32_t slots)
 {
-    if (ctx->lds_rec.p && ctx->lds_staged()) {
-        int cus = 0;
-        HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
-        ip.parts = 1u;
-        if (ctx->lds_kind == kLdsIndexed)
-            hipLaunchKernelGGL(hase_importance_staged_kernel<kLdsIndexed>, dim3((uint32_t)std::max(1, cus)),
-                               dim3(kStagedBlock), 0, ctx->stream, ip);
-        else
-            hipLaunchKernelGGL(hase_importance_staged_kernel<kLdsCompact>, dim3((uint32_t)std::max(1, cus)),
-                               dim3(kStagedBlock), 0, ctx->stream, ip);
-        HIP_CHECK(hipGetLastError());
-        if (!ip.transfer) {
-            hipLaunchKernelGGL(hase_prefix_kernel, dim3(slots), dim3(kBlock), 0, ctx->stream, ip);
-            HIP_CHECK(hipGetLastError());
+    const uint32_t T = ctx->T;
+    int cus = 0;
+    HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+    const uint32_t wide = (uint32_t)std::max(1, cus) * 8u;   // a multiple of the 8 XCDs
+    const uint64_t tiles = (uint64_t)slots * ((T + kTilePaths - 1u) / kTilePaths);
+    PathParams q{};
+    q.p = ip;
+    q.rows = std::min(ctx->path_cap, kPathEntries - 1u) + 1u;
+    // the list numbers paths in 32 bits
+    const uint64_t held = (uint64_t)slots * T <= 0xFFFFFFFFull ? reserve_paths(ctx, tiles, (size_t)slots * T) : 0u;
+    if (held) {
+        HIP_CHECK(hipMemsetAsync(ctx->path_count.p, 0, sizeof(uint32_t), ctx->stream));
+        q.path = ctx->path.p;
+        q.head = reinterpret_cast<PathHead*>(ctx->path_head.p);
+        q.over = ctx->path_over.p;
+        q.over_count = ctx->path_count.p;
+        q.inv_layers = ip.m.layers > 1u ? (uint32_t)(((1ull << 32) + ip.m.layers - 1u) / ip.m.layers) : 0u;
+        for (q.tile0 = 0; q.tile0 < tiles; q.tile0 += q.ntiles) {
+            q.ntiles = (uint32_t)std::min<uint64_t>(held, tiles - q.tile0);
+            const dim3 walk((q.ntiles + kBlock / 64 - 1) / (kBlock / 64));
+            hipLaunchKernelGGL(hase_column_path_kernel, walk, dim3(kBlock), 0, ctx->stream, q);
+            const dim3 grid(std::min<uint32_t>((uint32_t)std::max(1, cus) * (2048u / kMapBlock), (q.ntiles + 7u) / 8u * 8u));
+            hipLaunchKernelGGL(hase_column_map_kernel, grid, dim3(kMapBlock), 0, ctx->stream, q);
         }
-        return;
     }
-    // a small batch would leave most of the chip idle: split each sample's walks
-    ip.parts = importance_parts(ctx, slots);
-    if (ctx->lds_rec.p && ctx->lds_kind == kCompactGlobal)
-        hipLaunchKernelGGL(hase_importance_kernel<kCompactGlobal>, dim3(slots * ip.parts), dim3(kBlock), 0,
-                           ctx->stream, ip);
-    else
-        hipLaunchKernelGGL(hase_importance_kernel<0u>, dim3(slots * ip.parts), dim3(kBlock), 0, ctx->stream, ip);
+    const dim3 list(held ? wide / 8u : wide);
+    hipLaunchKernelGGL(hase_column_list_kernel, list, dim3(kBlock), 0, ctx->stream, q);
     HIP_CHECK(hipGetLastError());
-    if (ip.parts > 1u && !ip.transfer) {
+    if (!ip.transfer) {
         hipLaunchKernelGGL(hase_prefix_kernel, dim3(slots), dim3(kBlock), 0, ctx->stream, ip);
         HIP_CHECK(hipGetLastError());
     }
@@ -1292,6 +1324,7 @@ void build_proposal(hase_context* ctx, uint32_t b0, const uint32_t* sample_of, u
         launch_importance(ctx, ip, slots);
         tm.imp.emplace_back(i0, record(ctx));
         ctx->stats.importance_launches++;
+        ctx->stats.importance_walks += (uint64_t)slots * R * ctx->P;
     }
 
 }
@@ -1519,7 +1552,6 @@ void evaluate(hase_context* ctx, hase_result_t* res)
     HIP_CHECK(hipMemcpy(cnt, ctx->counters.p, sizeof(cnt), hipMemcpyDeviceToHost));
     ctx->stats.rays = cnt[0];
     ctx->stats.ray_steps = cnt[1];
-    ctx->stats.importance_walks = cnt[2];
     ctx->stats.importance_steps = cnt[3];
     uint64_t dropped = 0;
     for (uint32_t s = first; s <= last; ++s)
@@ -1636,7 +1668,7 @@ void batch_evaluate(hase_batch* b, hase_result_t* const* results)
         hase_context* ctx = b->ctx[p];
         const hase_tuning_t& ct = ctx->tuning;
         const uint32_t count = ctx->comp.max_sample_range - ctx->comp.min_sample_range + 1u;
-        solo[p] = ctx->lds_rec.p != nullptr && ctx->lds_staged() && ct.mode == HASE_TRACE_QUEUE && ct.stage_lds &&
+        solo[p] = ctx->lds_staged() && ct.mode == HASE_TRACE_QUEUE && ct.stage_lds &&
                   ct.refill_lanes == 0u &&
                   count >= kSoloSamples;
         if (!solo[p]) continue;
@@ -1799,10 +1831,7 @@ void batch_evaluate(hase_batch* b, hase_result_t* const* results)
         qs.refill = tu.refill_lanes;
         qs.budget = tu.step_budget;
         b->generation++;   // buffers may have moved: capture again
-        bool table_compact = true;
-        for (size_t w = 0; w < part.size(); ++w) table_compact = table_compact && table[w].m.cmp_rec != nullptr;
-        queue_ms += queue_run(b->stream, b->device, tu, qs, total, rounds, b->graph, b->generation, nullptr,
-                              table_compact);
+        queue_ms += queue_run(b->stream, b->device, tu, qs, total, rounds, b->graph, b->generation);
         b->stats.trace_launches += rounds;
         std::vector<float> h_phi(total);
         std::vector<double> h_mse(total), h_se(total);
@@ -1866,7 +1895,7 @@ void batch_evaluate(hase_batch* b, hase_result_t* const* results)
         HIP_CHECK(hipMemcpy(c2, ctx->counters.p, sizeof(c2), hipMemcpyDeviceToHost));
         b->stats.rays += c2[0];
         b->stats.ray_steps += c2[1];
-        b->stats.importance_walks += c2[2];
+        b->stats.importance_walks += ctx->stats.importance_walks;
         b->stats.importance_steps += c2[3];
         b->stats.importance_launches += ctx->stats.importance_launches;
         uint64_t dr = 0;
@@ -1939,10 +1968,10 @@ void autotune(hase_context* ctx, uint32_t probe, hase_tuning_t* best)
         };
         if (ctx->lds_rec.p) {
             // one work-group per CU holds a staged mesh: try it with the largest
-            // block (compact records in global memory keep the block size)
+            // block
             hase_tuning_t t = cur;
             t.stage_lds = cur.stage_lds ? 0u : 1u;
-            t.block_size = t.stage_lds && ctx->lds_staged() ? 1024u : cur.block_size;
+            t.block_size = t.stage_lds ? 1024u : cur.block_size;
             const double ms = time_it(t);
             if (ms < 0.98 * best_ms) {
                 best_ms = ms;

@@ -33,30 +33,69 @@ HASE_HD inline float bits_to_float(uint32_t u) { return __builtin_bit_cast(float
 // bits 0-30 (all ones at the boundary) and this triangle's cladding flag in
 // bit 31, so every neighbour word read also tells the walk what its current
 // triangle is made of.
-// Compact records, 32 B per triangle for staging the mesh in LDS:
+// Two smaller forms of the same words follow.  No kernel reads them any more;
+// the host checks hold walk_ray over them against the 48-byte records.
+// Compact records, 32 B per triangle:
 //   {x0, y0, x1, y1}  {x2, y2, W & 0xFFFFFFFF, W >> 32}
 // with W = f0 | f1 << 21 | f2 << 42 | cladding << 63 and f_k = neighbour << 2 |
 // shared edge (21 bits: neighbour < 2^19) or 0x1FFFFF at the boundary.
-// Indexed records, for meshes beyond kLdsTriangles: 16 B per triangle,
+// Indexed records, 16 B per triangle:
 //   {v0 | v1 << 16, v2 | cladding << 31, W & 0xFFFFFFFF, W >> 32}
 // with v_k the point index of vertex k (< 2^16) and W as above, followed by
 // the vertex table, the FP32 (x, y) of every mesh point, two per 16 bytes.
-// One more LDS read per new vertex than the compact records, but a Delaunay
-// disk (about T / 2 points) fits up to ~8,100 triangles instead of 4800.
-constexpr uint32_t kLdsTriangles = 4800;     // compact records: 150 KiB of LDS
 constexpr uint32_t kLdsStageWords = 10176;   // 16-byte words of LDS a staged kernel holds (159 KiB)
 constexpr uint32_t kLdsCompact = 1u, kLdsIndexed = 2u;
-// Meshes that fit neither LDS format keep the compact records in global
-// memory: the walk reads one vertex and one neighbour word per step from
-// them (two loads, 32 B per triangle) instead of three loads from the
-// 48-byte records.
-constexpr uint32_t kCompactGlobal = 3u;
+// Edge records: what a walk needs on entering triangle t through its edge f,
+// with N the vertex opposite f: N's coordinates, the links behind the two
+// other edges, R-N (edge f + 1, taken when N is left of the line) and N-L
+// (edge f + 2), and t's cladding flag.  A link names the next record, so a
+// step reads one record and decodes little; all ones mark the mesh boundary.
+//   global        16 B {x, y, left, right}, record 4 t + f; a link is the next
+//                 record's byte offset, plus in bit 0 the cladding flag of t;
+//                 the boundary's top bit is set
+//   kLdsEdges     12 B {x, y, left | right << 15 | cladding << 31}, record
+//                 3 t + f: 36 B per triangle, up to ~4,500 triangles in LDS
+//   kLdsIndexedEdges  vertex table float2 [np], the same links u32 [3T], point
+//                 index u16 [3T] of N: 18 B per triangle and 8 B per point, up
+//                 to ~7,400 triangles of a Delaunay disk
+//   kLdsTwins     vertex table float2 [np], u16 [3T] link behind edge k |
+//                 cladding << 15, u16 [3T] point index of vertex k: 12 B per
+//                 triangle and 8 B per point, up to ~10,100 triangles; a step
+//                 picks the two links and the vertex by f (~8 instructions more)
+constexpr uint32_t kLdsEdges = 4u, kLdsIndexedEdges = 5u, kLdsTwins = 6u;
+
+// Unsigned division by a divisor fixed per mesh, exact for every n (Granlund
+// and Montgomery, "Division by invariant integers using multiplication", PLDI
+// 1994, figure 4.1).
+struct FastDiv {
+    uint32_t mul, shift1, shift2;
+    HASE_HD uint32_t operator()(uint32_t n) const
+    {
+#if defined(__HIP_DEVICE_COMPILE__)
+        const uint32_t t = __umulhi(mul, n);
+#else
+        const uint32_t t = (uint32_t)(((uint64_t)mul * n) >> 32);
+#endif
+        return (t + ((n - t) >> shift1)) >> shift2;
+    }
+};
+
+inline FastDiv fast_div(uint32_t d)
+{
+    uint32_t l = 0;
+    while (l < 32u && (1ull << l) < d) ++l;
+    FastDiv f;
+    f.mul = (uint32_t)(((1ull << 32) * ((1ull << l) - d)) / d + 1ull);
+    f.shift1 = l < 1u ? l : 1u;
+    f.shift2 = l > 1u ? l - 1u : 0u;
+    return f;
+}
 
 struct MeshDev {
     const uint4* rec;      // 3 records per triangle
-    const uint4* lds_rec;  // records of kind lds_kind (staged in LDS, or read from global memory), or null
-    uint32_t lds_kind;     // 0: none, kLdsCompact, kLdsIndexed, kCompactGlobal
-    const uint4* cmp_rec;  // the compact records in global memory (meshes below 2^19 triangles), or null
+    const uint4* edges;    // edge records in global memory: 4 t + f
+    const uint4* lds_rec;  // edge records of kind lds_kind, to be staged in LDS, or null
+    uint32_t lds_kind;     // 0: none, kLdsEdges, kLdsIndexedEdges, kLdsTwins
     uint32_t lds_words;    // 16-byte words to stage
     const float* beta;     // [P] level-major: t + l * T, zero in cladding prisms
     const float* beta_col; // [P] column-major: t * layers + l, zero in cladding prisms
@@ -65,6 +104,7 @@ struct MeshDev {
     float nin_b, nout_b, nin_t, nout_t;
     int has_nidx;
     uint32_t T, layers, np;
+    FastDiv by_T, by_P;    // division by T and by T * layers
     float h, clad_alpha;
     float steps_per_cm;    // estimated triangle crossings per cm of xy path (1.2 sqrt(T / mesh area))
 };
@@ -129,6 +169,20 @@ HASE_HD inline uint32_t mul24(uint32_t a, uint32_t b)
     return __umul24(a, b);
 #else
     return a * b;
+#endif
+}
+
+// kFactor * a for a < 2^24: left to itself the compiler turns it into the
+// 32-bit multiply, a quarter of the rate, where it cannot see a's range.
+template <uint32_t kFactor>
+HASE_HD inline uint32_t mul24_by(uint32_t a)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    uint32_t r;
+    asm("v_mul_u32_u24_e32 %0, %2, %1" : "=v"(r) : "v"(a), "n"(kFactor));
+    return r;
+#else
+    return kFactor * a;
 #endif
 }
 
@@ -208,7 +262,7 @@ struct GlobalTriangles {
     }
 };
 
-// From the 32-byte compact records staged in LDS; the end point is
+// From the 32-byte compact records; the end point is
 // identified by its stored FP32 coordinates (ex, ey), which equal the
 // corners' of the same mesh point bit for bit.
 struct LdsTriangles {
@@ -251,7 +305,7 @@ struct LdsTriangles {
     }
 };
 
-// From the 16-byte indexed records and the vertex table staged in LDS
+// From the 16-byte indexed records and the vertex table
 // (vtx = the table, right after the T records); words, decoders and the end
 // test are those of the compact records.
 struct LdsIndexedTriangles : LdsTriangles {
@@ -283,7 +337,7 @@ struct LdsIndexedTriangles : LdsTriangles {
     }
 };
 
-// Fetch of records staged in LDS at s (kind kLdsCompact or kLdsIndexed: T
+// Fetch of records at s (kind kLdsCompact or kLdsIndexed: T
 // records, then the indexed format's vertex table).
 template <uint32_t kKind>
 using StagedFetch = std::conditional_t<kKind == kLdsIndexed, LdsIndexedTriangles, LdsTriangles>;
@@ -295,6 +349,149 @@ HASE_HD inline StagedFetch<kKind> staged_fetch(const uint4* s, uint32_t T)
         return LdsIndexedTriangles{{s}, reinterpret_cast<const float2*>(s + T)};
     else
         return LdsTriangles{s};
+}
+
+// Edge records by format: vertex(m, t, v); out(m, t, k), the link behind edge
+// k of a start triangle; enter(m, link, t, n, l), the step into the triangle
+// behind a link, with pick(l, left) the next link and clad(l) its flag.
+struct GlobalEdges {
+    using Links = uint2;
+    static constexpr uint32_t kNone = 0x80000000u;
+    HASE_HD static bool boundary(uint32_t w) { return (int32_t)w < 0; }
+    HASE_HD static uint32_t clad(const Links& l) { return l.x & 1u; }
+    HASE_HD static uint32_t pick(const Links& l, bool left) { return left ? l.x : l.y; }
+    HASE_HD static uint4 at(const MeshDev& m, uint32_t offset)
+    {
+        return *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(m.edges) + offset);
+    }
+    HASE_HD float2 vertex(const MeshDev& m, uint32_t t, uint32_t v) const
+    {
+        const uint32_t i = 4u * t + (v == 2u ? 0u : v + 1u);
+        return *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(m.edges) + i * 16u);
+    }
+    HASE_HD uint32_t out(const MeshDev& m, uint32_t t, uint32_t k, uint32_t& own) const
+    {
+        const uint4 q = at(m, (4u * t + (k == 0u ? 2u : k - 1u)) * 16u);
+        own = q.z & 1u;
+        return q.z;
+    }
+    HASE_HD void enter(const MeshDev& m, uint32_t w, uint32_t& t, float2& n, Links& l) const
+    {
+        const uint4 q = at(m, w & ~15u);
+        t = w >> 6;
+        n = make_float2(bits_to_float(q.x), bits_to_float(q.y));
+        l = make_uint2(q.z, q.w);
+    }
+};
+
+// Links of the LDS formats: 15-bit record numbers 3 t + f.
+struct ShortLinks {
+    using Links = uint32_t;
+    static constexpr uint32_t kNone = 0x7FFFu;
+    HASE_HD static bool boundary(uint32_t w) { return w == kNone; }
+    HASE_HD static uint32_t clad(Links l) { return l >> 31; }
+    HASE_HD static uint32_t pick(Links l, bool left)
+    {
+        const uint32_t shift = left ? 0u : 15u;
+        return (l >> shift) & kNone;
+    }
+    // i / 3 for i < 2^16
+    HASE_HD static uint32_t third(uint32_t i) { return mul24_by<43691u>(i) >> 17; }
+};
+
+struct LdsEdge {
+    float x, y;
+    uint32_t links;
+};
+
+struct LdsEdges : ShortLinks {
+    const LdsEdge* rec;
+    HASE_HD float2 vertex(const MeshDev&, uint32_t t, uint32_t v) const
+    {
+        const LdsEdge& e = rec[3u * t + (v == 2u ? 0u : v + 1u)];
+        return make_float2(e.x, e.y);
+    }
+    HASE_HD uint32_t out(const MeshDev&, uint32_t t, uint32_t k, uint32_t& own) const
+    {
+        const uint32_t l = rec[3u * t + (k == 0u ? 2u : k - 1u)].links;
+        own = clad(l);
+        return pick(l, true);
+    }
+    HASE_HD void enter(const MeshDev&, uint32_t w, uint32_t& t, float2& n, Links& l) const
+    {
+        const LdsEdge& e = *reinterpret_cast<const LdsEdge*>(reinterpret_cast<const char*>(rec) + mul24_by<12u>(w));
+        n = make_float2(e.x, e.y);
+        l = e.links;
+        t = third(w);
+    }
+};
+
+struct LdsIndexedEdges : ShortLinks {
+    const float2* vtx;
+    const uint32_t* link;
+    const uint16_t* opp;   // point index of N
+    HASE_HD float2 vertex(const MeshDev&, uint32_t t, uint32_t v) const
+    {
+        return vtx[opp[3u * t + (v == 2u ? 0u : v + 1u)]];
+    }
+    HASE_HD uint32_t out(const MeshDev&, uint32_t t, uint32_t k, uint32_t& own) const
+    {
+        const uint32_t l = link[3u * t + (k == 0u ? 2u : k - 1u)];
+        own = clad(l);
+        return pick(l, true);
+    }
+    HASE_HD void enter(const MeshDev&, uint32_t w, uint32_t& t, float2& n, Links& l) const
+    {
+        n = vtx[opp[w]];
+        l = link[w];
+        t = third(w);
+    }
+};
+
+struct LdsTwins : ShortLinks {
+    const float2* vtx;
+    const uint16_t* twin;   // link behind edge k of t: 3 t + k
+    const uint16_t* point;  // point index of vertex k of t: 3 t + k
+    HASE_HD float2 vertex(const MeshDev&, uint32_t t, uint32_t v) const { return vtx[point[3u * t + v]]; }
+    HASE_HD uint32_t out(const MeshDev&, uint32_t t, uint32_t k, uint32_t& own) const
+    {
+        const uint32_t w = twin[3u * t + k];
+        own = w >> 15;
+        return w & kNone;
+    }
+    HASE_HD static uint32_t clad(Links l) { return l >> 31; }
+    HASE_HD static uint32_t pick(Links l, bool left) { return (left ? l : l >> 16) & kNone; }
+    HASE_HD void enter(const MeshDev&, uint32_t w, uint32_t& t, float2& n, Links& l) const
+    {
+        t = third(w);
+        const uint32_t f = w - 3u * t;
+        const uint32_t e1 = f == 2u ? w - 2u : w + 1u, e2 = f == 0u ? w + 2u : w - 1u;
+        n = vtx[point[e2]];   // vertex f + 2
+        l = twin[e1] | (uint32_t)twin[e2] << 16;
+    }
+};
+
+// Edge records of kind kKind staged at s (0: the global ones).
+template <uint32_t kKind>
+using EdgeFetch = std::conditional_t<kKind == kLdsEdges, LdsEdges,
+                                     std::conditional_t<kKind == kLdsIndexedEdges, LdsIndexedEdges,
+                                                        std::conditional_t<kKind == kLdsTwins, LdsTwins, GlobalEdges>>>;
+
+template <uint32_t kKind>
+HASE_HD inline EdgeFetch<kKind> edge_fetch(const uint4* s, uint32_t T, uint32_t np)
+{
+    const float2* xy = reinterpret_cast<const float2*>(s);
+    if constexpr (kKind == kLdsEdges) {
+        return LdsEdges{{}, reinterpret_cast<const LdsEdge*>(s)};
+    } else if constexpr (kKind == kLdsIndexedEdges) {
+        const uint32_t* link = reinterpret_cast<const uint32_t*>(xy + np);
+        return LdsIndexedEdges{{}, xy, link, reinterpret_cast<const uint16_t*>(link + 3u * T)};
+    } else if constexpr (kKind == kLdsTwins) {
+        const uint16_t* twin = reinterpret_cast<const uint16_t*>(xy + np);
+        return LdsTwins{{}, xy, twin, twin + 3u * T};
+    } else {
+        return GlobalEdges{};
+    }
 }
 
 // Exit edge among the candidates s_k (edge k joins corners k and k+1): its
@@ -385,6 +582,20 @@ HASE_HD inline float along(float dx, float dy, float x, float y) { return dx * x
 HASE_HD inline float edge_sigma(float cl, float wl, float cr, float wr, float inv_d2)
 {
     return (cl * wr - cr * wl) * inv_d2 * fast_rcp(cl - cr);
+}
+
+// max(min(a, b, 1), sig) for sig <= 1 and at most one of a, b not a number
+// (then the other counts); the instructions by hand, as fminf first copies
+// each operand that the compiler cannot prove quiet.
+HASE_HD inline float next_sigma(float a, float b, float sig)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    float s;
+    asm("v_min_f32_e32 %0, %1, %2" : "=v"(s) : "v"(a), "v"(b));
+    return __builtin_amdgcn_fmed3f(s, sig, 1.0f);
+#else
+    return fmaxf(fminf(fminf(a, b), 1.0f), sig);
+#endif
 }
 
 template <bool kReflect>
@@ -597,6 +808,139 @@ HASE_HD inline WalkOut walk_ray(const MeshDev& m, float ax, float ay, float za, 
 {
     return walk_ray(m, ax, ay, za, t, layer, fetch.vertex(m, t, 0u), fetch.vertex(m, t, 1u), fetch.vertex(m, t, 2u),
                     ex, ey, ze, nrefl, first, fetch);
+}
+
+// Whole walk of one ray over edge records: walk_begin and walk_advance
+// operation for operation, with the next level plane, the layer's offset into
+// beta and the next copy boundary carried from crossing to crossing instead of
+// being rebuilt from the layer, copy and direction at every step.  The loop
+// has one exit and tells the reasons apart behind it: with a break for each,
+// the compiler copied a dozen registers at every step (95 vector instructions
+// a step instead of 50).  Vector issue bounds the staged walks (89% of the
+// cycles); a 2060-point, 20-level disk with reflections and cladding takes
+// 40.3 ms for 5,000 samples from 36-byte edge records, 55 from the 32-byte
+// triangle records that walk_ray reads, a 5,000-point one 11.5 against 19.
+template <class Edges>
+HASE_HD inline WalkOut walk_edges(const MeshDev& m, float ax, float ay, float za, uint32_t t, uint32_t layer, float2 p0,
+                                  float2 p1, float2 p2, float ex, float ey, float ze, uint32_t nrefl, uint32_t first,
+                                  const Edges& edges)
+{
+    WalkOut o;
+    o.refl = 1.0f;
+    o.steps = 0u;
+    o.status = 0;
+    const float dx = ex - ax, dy = ey - ay, dzeta = ze - za, dz = dzeta * m.h;
+    const float D = sqrtf(dx * dx + dy * dy + dz * dz);
+    o.length = D;
+    if (!(D > 0.0f)) {
+        o.beta_len = o.gain_len = o.clad_len = 0.0f;
+        return o;
+    }
+    const float d2 = dx * dx + dy * dy;
+    const float inv_d2 = d2 > 0.0f ? 1.0f / d2 : 0.0f;
+    const float inv_dz = dzeta != 0.0f ? 1.0f / dzeta : 0.0f;
+    // exit of the start triangle: the edge whose start vertex is right of the
+    // line and whose end vertex is left of it (counter-clockwise order)
+    const float c0 = side_of(dx, dy, p0.x - ax, p0.y - ay), c1 = side_of(dx, dy, p1.x - ax, p1.y - ay);
+    const float c2 = side_of(dx, dy, p2.x - ax, p2.y - ay);
+    const bool b0 = c0 >= 0.0f, b1 = c1 >= 0.0f, b2 = c2 >= 0.0f;
+    int k = (!b0 && b1) ? 0 : (!b1 && b2) ? 1 : (!b2 && b0) ? 2 : -1;
+    if (k < 0) {
+        if (b0) {
+            k = (c0 <= c1 && c0 <= c2) ? 0 : (c1 <= c2 ? 1 : 2);
+        } else {
+            const int km = (c0 >= c1 && c0 >= c2) ? 0 : (c1 >= c2 ? 1 : 2);
+            k = km == 0 ? 2 : km - 1;
+        }
+    }
+    const float2 pr = k == 0 ? p0 : (k == 1 ? p1 : p2);
+    const float2 pl = k == 0 ? p1 : (k == 1 ? p2 : p0);
+    float cr = k == 0 ? c0 : (k == 1 ? c1 : c2);
+    float cl = k == 0 ? c1 : (k == 1 ? c2 : c0);
+    float wr = along(dx, dy, pr.x - ax, pr.y - ay);
+    float wl = along(dx, dy, pl.x - ax, pl.y - ay);
+    uint32_t own;
+    uint32_t link = edges.out(m, t, (uint32_t)k, own);
+    const bool at_end = (p0.x == ex && p0.y == ey) || (p1.x == ex && p1.y == ey) || (p2.x == ex && p2.y == ey) ||
+                        d2 == 0.0f;
+    float sxy = at_end ? 1.0f : edge_sigma(cl, wl, cr, wr, inv_d2);
+    float clad = (float)own;
+    // level planes, measured back from the end: the next one and the next
+    // copy boundary minus the end's; a level ray (inv_dz = 0) meets none
+    const float up = dzeta > 0.0f ? 1.0f : -1.0f;
+    float pm = (float)((int)layer + (dzeta > 0.0f ? 1 : 0)) - ze;
+    float pb = (dzeta > 0.0f ? (float)m.layers : 0.0f) - ze;
+    float sz = fmaf(pm, inv_dz, 1.0f);
+    uint32_t lvl = mul24(layer, m.T), dir = dzeta > 0.0f ? m.T : 0u - m.T;
+    float sig = 0.0f, beta_sig = 0.0f, clad_sig = 0.0f;
+    uint32_t applied = 0u, it = 0u;
+    for (;;) {
+        // used at the end of the step only: the load runs beside the step into
+        // the next triangle (zero in cladding prisms)
+        const float beta = load_f32(m.beta, t + lvl);
+        const bool cross = !(sz <= sxy);
+        const float snext = next_sigma(sxy, sz, sig);
+        const float seg = snext - sig;
+        clad_sig = fmaf(clad, seg, clad_sig);
+        sig = snext;
+        ++it;
+        const bool done = (int)(sig >= 1.0f) | ((int)cross & (int)Edges::boundary(link)) | (int)(it == kMaxSteps);
+        if (!done) {
+            if (!cross) {
+                lvl += dir;
+                if (pm == pb) {
+                    // at a copy boundary the ray stays in the layer and turns (a
+                    // direct ray ends before it meets one)
+                    lvl -= dir;
+                    if (applied < nrefl) {
+                        const float vz = dz / D;
+                        o.refl *= surface_factor(m, t, (int)dir < 0 ? 0u : 1u, fmaxf(0.0f, 1.0f - vz * vz));
+                        ++applied;
+                    }
+                    dir = 0u - dir;
+                    pb = fmaf(up, (float)m.layers, pb);
+                }
+                pm += up;
+                sz = fmaf(pm, inv_dz, 1.0f);
+            } else {
+                float2 pn;
+                typename Edges::Links links;
+                edges.enter(m, link, t, pn, links);
+                const float X = pn.x - ax, Y = pn.y - ay;
+                const float c = side_of(dx, dy, X, Y), a = along(dx, dy, X, Y);
+                const bool left = c >= 0.0f;
+                // left of the line: leave through R-N, N becomes L; else through N-L
+                cl = left ? c : cl;
+                wl = left ? a : wl;
+                cr = left ? cr : c;
+                wr = left ? wr : a;
+                link = Edges::pick(links, left);
+                clad = (float)Edges::clad(links);
+                const bool end = (pn.x == ex) & (pn.y == ey);
+                sxy = end ? 1.0f : edge_sigma(cl, wl, cr, wr, inv_d2);
+            }
+        }
+        beta_sig = fmaf(beta, seg, beta_sig);
+        if (done) break;
+    }
+    // leaving the mesh sideways: only rounding short of the end (a sample
+    // point on the rim) counts as arrival
+    if (sig < 1.0f) {
+        const bool outside = !(sz <= sxy) && Edges::boundary(link);
+        o.status = !outside ? 2 : (1.0f - sig) * D > 2e-5f * (1.0f + D) ? 1 : 0;
+    }
+    o.steps = it;
+    if (sig >= 1.0f && applied < nrefl) {
+        // an end point on a reflecting plane takes its last factors here
+        const float vz = dz / D;
+        const float sin2 = fmaxf(0.0f, 1.0f - vz * vz);
+        for (; applied < nrefl; ++applied)
+            o.refl *= surface_factor(m, t, (applied & 1u) ? 1u - first : first, sin2);
+    }
+    o.beta_len = beta_sig * D;
+    o.gain_len = (sig - clad_sig) * D;
+    o.clad_len = clad_sig * D;
+    return o;
 }
 
 // Height, in layer units, of the mirror image of a sample point on plane

@@ -122,9 +122,8 @@ struct ItemCtx {
     SampleGeom sp;
     const double* pre;
     const uint32_t* bk;       // prefix buckets of the item's sample
-    size_t n;
     double Q, U, scale;
-    uint32_t sample, launch, r0, seed;
+    uint32_t n, sample, launch, r0, seed;
 };
 
 // Start point, start triangle's corners, end image and proposal probability
@@ -137,17 +136,32 @@ struct RayStart {
 
 // Proposal entry of ray `ray` of an item: the first entry whose prefix
 // exceeds the ray's systematic target, searched between the target's buckets.
-__device__ __forceinline__ size_t ray_entry(const ItemCtx& c, uint32_t ray)
+__device__ __forceinline__ uint32_t ray_entry(const ItemCtx& c, uint32_t ray)
 {
     const double target = ((double)ray + c.U) * c.scale;
     const double kt = target * (double)kPrefixBuckets;
     const uint32_t kb = kt >= (double)(kPrefixBuckets - 1u) ? kPrefixBuckets - 1u : (uint32_t)kt;
-    size_t lo = c.bk[kb], hi = (kb + 1u < kPrefixBuckets ? (size_t)c.bk[kb + 1u] : c.n - 1) + 1;
+    uint32_t lo = c.bk[kb], hi = (kb + 1u < kPrefixBuckets ? c.bk[kb + 1u] : c.n - 1u) + 1u;
     while (lo < hi) {
-        const size_t mid = (lo + hi) >> 1;
-        if (c.pre[mid] > target) hi = mid; else lo = mid + 1;
+        const uint32_t mid = lo + ((hi - lo) >> 1);
+        if (c.pre[mid] > target) hi = mid; else lo = mid + 1u;
     }
-    return lo < c.n ? lo : c.n - 1;
+    return lo < c.n ? lo : c.n - 1u;
+}
+
+// Slice, prism, triangle and layer of a proposal entry.
+struct EntryParts {
+    uint32_t k, j, t, l;
+};
+
+__device__ __forceinline__ EntryParts entry_parts(const MeshDev& m, uint32_t e)
+{
+    EntryParts p;
+    p.k = m.by_P(e);
+    p.j = e - p.k * (m.T * m.layers);
+    p.l = m.by_T(p.j);
+    p.t = p.j - mul24(p.l, m.T);
+    return p;
 }
 
 // Estimated prism steps of a ray from entry e to the item's sample: triangle
@@ -155,26 +169,23 @@ __device__ __forceinline__ size_t ray_entry(const ItemCtx& c, uint32_t ray)
 // plus the level planes between the start layer's middle and the end image.
 // Only used to order the rays of a wavefront (longer walks together).
 template <class Fetch>
-__device__ __forceinline__ float ray_steps_estimate(const MeshDev& m, const ItemCtx& c, size_t e, const Fetch& fetch)
+__device__ __forceinline__ float ray_steps_estimate(const MeshDev& m, const ItemCtx& c, uint32_t e, const Fetch& fetch)
 {
-    const uint32_t T = m.T, P = T * m.layers;
-    const uint32_t k = (uint32_t)(e / P), j = (uint32_t)(e % P);
-    const uint32_t t = j % T, l = j / T;
-    const float2 p0 = fetch.vertex(m, t, 0u);
-    const float ez = (float)image_plane(c.sp.plane, (int)m.layers, (k + 1u) >> 1, k & 1u);
+    const EntryParts p = entry_parts(m, e);
+    const float2 p0 = fetch.vertex(m, p.t, 0u);
+    const float ez = (float)image_plane(c.sp.plane, (int)m.layers, (p.k + 1u) >> 1, p.k & 1u);
     const float dx = p0.x - c.sp.px, dy = p0.y - c.sp.py;
-    return sqrtf(dx * dx + dy * dy) * m.steps_per_cm + fabsf((float)l + 0.5f - ez);
+    return __builtin_amdgcn_sqrtf(dx * dx + dy * dy) * m.steps_per_cm + fabsf((float)p.l + 0.5f - ez);
 }
 
 template <class Fetch>
-__device__ __forceinline__ RayStart draw_ray_at(const MeshDev& m, const ItemCtx& c, uint32_t ray, size_t e, double& q,
+__device__ __forceinline__ RayStart draw_ray_at(const MeshDev& m, const ItemCtx& c, uint32_t ray, uint32_t e, double& q,
                                                 uint32_t& jout, const Fetch& fetch)
 {
-    const uint32_t T = m.T, P = T * m.layers;
-    q = c.pre[e] - (e ? c.pre[e - 1] : 0.0);
-    const uint32_t k = (uint32_t)(e / P), j = (uint32_t)(e % P);
-    const uint32_t t = j % T, l = j / T;
-    jout = j;
+    q = c.pre[e] - (e ? c.pre[e - 1u] : 0.0);
+    const EntryParts parts = entry_parts(m, e);
+    const uint32_t t = parts.t, l = parts.l, k = parts.k;
+    jout = parts.j;
     uint32_t rnd[4];
     philox4x32_10(ray, c.sample, c.launch, kTagRay, c.seed, kKeyTag, rnd);
     float u1 = u32_to_unit(rnd[0]), u2 = u32_to_unit(rnd[1]), u3 = u32_to_unit(rnd[2]);
@@ -208,27 +219,63 @@ __device__ __forceinline__ void start_ray(const MeshDev& m, const ItemCtx& c, ui
     walk_begin(m, lr.w, r.ax, r.ay, r.az, r.t, r.l, r.p0, r.p1, r.p2, c.sp.px, c.sp.py, r.ez, r.nr, r.fp, fetch);
 }
 
+// Problem constants of the device table, read through the scalar cache (the
+// table is constant for the launch and the address uniform in the wavefront)
+// and with their pointers known to be global, so that they cost the walks no
+// vector registers and no generic-address loads.
+// written by earlier kernels only, indexed uniformly: read through the scalar cache
+typedef const __attribute__((address_space(4))) uint32_t ConstU32;
+
+template <class T>
+__device__ __forceinline__ void as_global(T*& p)
+{
+    p = (T*)(__attribute__((address_space(1))) T*)(uintptr_t)p;
+}
+
+__device__ __forceinline__ ProblemDev table_problem(const ProblemDev* at)
+{
+    typedef const __attribute__((address_space(4))) uint64_t ConstU64;
+    constexpr uint32_t kWords = sizeof(ProblemDev) / 8u;
+    static_assert(sizeof(ProblemDev) % 8u == 0u && alignof(ProblemDev) == 8u, "read as 64-bit words");
+    uint64_t w[kWords];
+    ConstU64* from = (ConstU64*)at;
+#pragma unroll
+    for (uint32_t i = 0; i < kWords; ++i) w[i] = from[i];
+    ProblemDev pd;
+    __builtin_memcpy(&pd, w, sizeof(pd));
+    as_global(pd.m.rec);
+    as_global(pd.m.edges);
+    as_global(pd.m.beta);
+    as_global(pd.m.bv);
+    as_global(pd.m.refl);
+    as_global(pd.pts);
+    as_global(pd.prefix);
+    as_global(pd.Q);
+    as_global(pd.buckets);
+    as_global(pd.sample_of);
+    return pd;
+}
+
 //
 // kTable: per-problem constants from the device table (batches of several
 // problems); otherwise from the kernel argument `one` (a single problem), so
-// they sit in scalar registers.  kLds (single problem whose records fit in
-// LDS: kLdsCompact or kLdsIndexed, 0 for none): the work-group first copies
-// the staged triangle records into LDS and the walks read them there; beta
-// stays in global memory.  kCompactGlobal: the walks read the compact
-// records of the item's problem from global memory (single problems too
-// large for LDS, and the problem table of a batch).
-template <bool kRefill, bool kTable, uint32_t kLds>
+// they sit in scalar registers.  kKind (single problem whose edge records fit
+// in LDS: kLdsEdges, kLdsIndexedEdges or kLdsTwins): the work-group first
+// copies them into LDS and the walks read them there; beta stays in global
+// memory.  0: the walks read the item's problem's records from global memory
+// (the lane-refill variant the 48-byte ones).
+template <bool kRefill, bool kTable, uint32_t kKind>
 __global__ void __launch_bounds__(kQueueMaxBlock) hase_queue_trace_kernel(QueueState q, ProblemDev one)
 {
     const uint32_t n_active = q.scalars[kNActive];
     if (n_active == 0u) return;
-    const uint4* lds_rec = nullptr;
-    if constexpr (kLds == kLdsCompact || kLds == kLdsIndexed) {
+    const uint4* staged = nullptr;
+    if constexpr (kKind != 0u) {
         __shared__ uint4 s_tri[kLdsStageWords];
         const uint32_t n = one.m.lds_words;
         for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) s_tri[i] = one.m.lds_rec[i];
         __syncthreads();
-        lds_rec = s_tri;
+        staged = s_tri;
     }
     const uint32_t total = q.item_off[n_active];
     const int lane = threadIdx.x & 63;
@@ -243,25 +290,26 @@ __global__ void __launch_bounds__(kQueueMaxBlock) hase_queue_trace_kernel(QueueS
         const uint32_t last = min(total, first + q.queue_chunk);
         for (uint32_t item = first; item < last; ++item) {
             // listed slot of the item: last a with item_off[a] <= item
+            ConstU32* item_off = (ConstU32*)q.item_off;
             uint32_t lo = 0, hi = n_active;
             while (hi - lo > 1u) {
                 const uint32_t mid = (lo + hi) >> 1;
-                if (q.item_off[mid] <= item) lo = mid; else hi = mid;
+                if (item_off[mid] <= item) lo = mid; else hi = mid;
             }
-            const uint32_t slot = q.list[lo];
-            const ProblemDev& pd = kTable ? q.problems[q.slot_problem[slot]] : one;
-            const MeshDev m = pd.m;
+            const uint32_t slot = ((ConstU32*)q.list)[lo];
+            const ProblemDev pd = kTable ? table_problem(q.problems + ((ConstU32*)q.slot_problem)[slot]) : one;
+            const MeshDev& m = pd.m;
             const uint32_t local = slot - pd.slot0;
-            const uint32_t nrays = q.nrays[slot];
-            const uint32_t ir = q.item_rays[slot];
+            const uint32_t nrays = ((ConstU32*)q.nrays)[slot];
+            const uint32_t ir = ((ConstU32*)q.item_rays)[slot];
             ItemCtx c;
-            c.r0 = (item - q.item_off[lo]) * ir;
+            c.r0 = (item - item_off[lo]) * ir;
             const uint32_t cnt = min(ir, nrays - c.r0);
             c.sample = pd.sample_of ? pd.sample_of[local] : pd.sample_base + local;
-            c.launch = q.launch[slot];
+            c.launch = ((ConstU32*)q.launch)[slot];
             c.seed = pd.seed;
             c.sp = sample_point(pd.pts, m.np, c.sample);
-            c.n = pd.n;
+            c.n = (uint32_t)pd.n;
             const uint32_t own = pd.shared ? 0u : local;   // slot whose proposal the rays follow
             c.pre = pd.prefix + (size_t)own * pd.n;
             c.bk = pd.buckets + (size_t)own * kPrefixBuckets;
@@ -302,8 +350,8 @@ __global__ void __launch_bounds__(kQueueMaxBlock) hase_queue_trace_kernel(QueueS
                         key[r] = 0xFFFFFF00u | li;   // past the item's end: sorted last, skipped
                         ent[r] = 0u;
                         if (g0 + li < cnt) {
-                            const size_t e = ray_entry(c, c.r0 + g0 + li);
-                            ent[r] = (uint32_t)e;
+                            const uint32_t e = ray_entry(c, c.r0 + g0 + li);
+                            ent[r] = e;
                             const float est = fminf(ray_steps_estimate(m, c, e, fetch) * 16.0f, 16777214.0f);
                             key[r] = ((uint32_t)est << 8) | li;
                         }
@@ -332,23 +380,16 @@ __global__ void __launch_bounds__(kQueueMaxBlock) hase_queue_trace_kernel(QueueS
                         if (g0 + li < cnt) {
                             double qprob;
                             uint32_t j;
-                            const RayStart s = draw_ray_at(m, c, c.r0 + g0 + li, (size_t)mine[0], qprob, j, fetch);
-                            const WalkOut w = walk_ray(m, s.ax, s.ay, s.az, s.t, s.l, s.p0, s.p1, s.p2, c.sp.px,
-                                                       c.sp.py, s.ez, s.nr, s.fp, fetch);
+                            const RayStart s = draw_ray_at(m, c, c.r0 + g0 + li, mine[0], qprob, j, fetch);
+                            const WalkOut w = walk_edges(m, s.ax, s.ay, s.az, s.t, s.l, s.p0, s.p1, s.p2, c.sp.px,
+                                                         c.sp.py, s.ez, s.nr, s.fp, fetch);
                             finish(w, qprob, j);
                         }
                         rays4 >>= 8;
                         mine[0] = mine[1]; mine[1] = mine[2]; mine[2] = mine[3];
                     }
                 };
-                for (uint32_t g0 = 0; g0 < cnt; g0 += 256u) {
-                    if constexpr (kLds != 0u) {
-                        // staged records, or the item's problem's compact records in global memory
-                        run_group(g0, staged_fetch<kLds>(kLds == kCompactGlobal ? m.cmp_rec : lds_rec, m.T));
-                    } else {
-                        run_group(g0, GlobalTriangles{});
-                    }
-                }
+                for (uint32_t g0 = 0; g0 < cnt; g0 += 256u) run_group(g0, edge_fetch<kKind>(staged, m.T, m.np));
             } else {
                 LaneRay lr;
                 bool have = (uint32_t)lane < cnt;
@@ -388,11 +429,9 @@ __global__ void __launch_bounds__(kQueueMaxBlock) hase_queue_trace_kernel(QueueS
             }
         }
     }
-    const unsigned long long ws = wave_sum_u64(steps), wr = wave_sum_u64(rays);
-    if (lane == 0 && wr) {
-        atomicAdd(&q.counters[0], wr);
-        atomicAdd(&q.counters[1], ws);
-    }
+    __shared__ unsigned long long red[2][kQueueMaxBlock / 64];
+    block_count(rays, red[0], &q.counters[0]);
+    block_count(steps, red[1], &q.counters[1]);
 }
 
 __global__ void hase_queue_finalize_kernel(QueueState q)
@@ -569,7 +608,7 @@ ProblemDev queue_problem(const hase_context* ctx, uint32_t slot0, uint32_t base,
 }
 
 float queue_run(hipStream_t stream, int device, const hase_tuning_t& tu, const QueueState& qs, uint32_t slots,
-                uint32_t rounds, GraphCache& gc, uint64_t generation, const ProblemDev* single, bool table_compact)
+                uint32_t rounds, GraphCache& gc, uint64_t generation, const ProblemDev* single)
 {
     int cus = 0, per = 0;
     HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
@@ -577,10 +616,9 @@ float queue_run(hipStream_t stream, int device, const hase_tuning_t& tu, const Q
     const bool table = single == nullptr;
     // LDS staging: single problem, no lane refill, mesh small enough
     const uint32_t lds = tu.stage_lds && !table && !refill && single->m.lds_rec != nullptr ? single->m.lds_kind : 0u;
-    auto kernel = lds == kLdsIndexed ? hase_queue_trace_kernel<false, false, kLdsIndexed>
-                : lds == kLdsCompact ? hase_queue_trace_kernel<false, false, kLdsCompact>
-                : lds == kCompactGlobal ? hase_queue_trace_kernel<false, false, kCompactGlobal>
-                : table && table_compact && tu.stage_lds && !refill ? hase_queue_trace_kernel<false, true, kCompactGlobal>
+    auto kernel = lds == kLdsEdges ? hase_queue_trace_kernel<false, false, kLdsEdges>
+                : lds == kLdsIndexedEdges ? hase_queue_trace_kernel<false, false, kLdsIndexedEdges>
+                : lds == kLdsTwins ? hase_queue_trace_kernel<false, false, kLdsTwins>
                 : refill ? (table ? hase_queue_trace_kernel<true, true, 0u> : hase_queue_trace_kernel<true, false, 0u>)
                          : (table ? hase_queue_trace_kernel<false, true, 0u> : hase_queue_trace_kernel<false, false, 0u>);
     HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, (int)tu.block_size, 0));

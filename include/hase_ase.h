@@ -343,9 +343,9 @@ typedef struct hase_tuning {
     uint32_t refill_lanes;    /* idle lanes that trigger a refill, 1..64; 0: each lane walks its rays to the end */
     uint32_t step_budget;     /* prism steps between refill checks, >= 1 */
     uint32_t use_graph;       /* 1: replay the rounds of a batch as a captured hipGraph */
-    uint32_t stage_lds;       /* 1: walk compact triangle records, staged in LDS when they fit (32-byte records
-                                 up to 4800 triangles, 16-byte indexed ones up to ~8,100), else read from
-                                 global memory; 0: the 48-byte global records (refill always uses these) */
+    uint32_t stage_lds;       /* 1: walk edge records staged in LDS when they fit (36 B per triangle up to ~4,500
+                                 triangles, smaller forms up to ~10,100), else read from global memory; 0: the
+                                 global edge records (refill always uses the 48-byte triangle records) */
     double probe_ms;          /* hase_context_autotune: device time of the chosen setting's probe */
 } hase_tuning_t;
 
