@@ -8,6 +8,9 @@
 
 namespace hase {
 
+// written by earlier kernels only, indexed uniformly: read through the scalar cache
+typedef const __attribute__((address_space(4))) uint32_t ConstU32;
+
 struct SampleGeom {
     float px, py;
     int plane;   // level of the sample point (its height in layer units)
@@ -51,15 +54,44 @@ __device__ __forceinline__ void block_count(unsigned long long v, unsigned long 
     }
 }
 
-// inclusive scan within a 64-lane wavefront
-__device__ __forceinline__ double wave_inclusive_scan(double v, int lane)
+// v of the lane that DPP control kCtrl names, 0.0 where it names none
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ double dpp_or_zero(double v)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, kCtrl, kRowMask, 0xF, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), kCtrl, kRowMask, 0xF, false);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
+// Inclusive scans of N values within a 64-lane wavefront, side by side so
+// that each hides the others' latency: shifts by 1, 2, 4 and 8 within rows of
+// 16 lanes, then the row ends broadcast to the next row (rows 1 and 3) and the
+// second row's end to the upper half.
+template <int N>
+__device__ __forceinline__ void wave_inclusive_scan(double (&v)[N])
 {
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        double o = __shfl_up(v, off, 64);
-        if (lane >= off) v += o;
-    }
-    return v;
+    for (int i = 0; i < N; ++i) v[i] += dpp_or_zero<0x111, 0xF>(v[i]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] += dpp_or_zero<0x112, 0xF>(v[i]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] += dpp_or_zero<0x114, 0xF>(v[i]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] += dpp_or_zero<0x118, 0xF>(v[i]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] += dpp_or_zero<0x142, 0xA>(v[i]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] += dpp_or_zero<0x143, 0xC>(v[i]);
+}
+
+// Lane 63's value in every lane
+__device__ __forceinline__ double wave_last(double v)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, 63);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), 63);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
 
 // Bitonic sort of a wavefront's 256 keys, ascending, key r * 64 + lane in

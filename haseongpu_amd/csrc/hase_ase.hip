@@ -48,143 +48,156 @@ using namespace hase;
 
 // Defensive-mixture proposal and its FP64 inclusive prefix for one sample
 // (one work-group): q_e = (1 - eps) imp_e / I + eps * bv_j / (R * Bsum), with
-// I the work-group sum of the thread partials `local`.  value(e) returns
-// imp_e and must be readable by every thread (the entries of other threads
-// are read after a barrier).  red holds kBlock/64 + 2 doubles of LDS.
-constexpr int kScanPer = 8;
+// I the sum of imp.  Entries e = (k * layers + l) * T + t are taken in rows of
+// 64 consecutive triangles of one layer and slice, so that a row's layer,
+// slice and addresses are uniform in the wavefront; value(k, l, t, bv) returns
+// imp_e.
+//
+// Each wavefront owns a run of rows and passes over it twice: first the sums
+// of imp and bv, whose prefix over the wavefronts is where each run starts;
+// then the entries again, each row scanned across the lanes and added to the
+// run's carry.  Nothing is exchanged inside a pass, so the loads of kRowsAhead
+// rows are in flight at a time and no wavefront waits for another.  (One run
+// for the work-group, 4096 entries at a time transposed through LDS with four
+// barriers, took 3.27 ms for 3,000 walked samples of 166,000 entries, 1.8
+// TB/s, and 6.4 ms for 6,000 learned ones; this takes 1.94 and 4.4, the latter
+// bound by the vector instructions of two evaluations per entry.)
+//
+// A run's last entry is set to the start of the next run and the others are
+// held below it, so that the prefix ascends and the buckets leave no gap where
+// the two passes round differently.
+constexpr uint32_t kRowsAhead = 4;
+constexpr uint32_t kPrefixMaxBlock = 1024;
 
-// (slice k, prism j = t + l*T) of a proposal entry e = k*P + j.
-struct EntryIndex {
-    uint32_t k, j, t, l;
-    __device__ __forceinline__ void init(uint32_t e, uint32_t P, uint32_t T)
+struct ProposalRow {
+    uint32_t tb, l, k, q;   // triangles 64 tb.., layer, slice, q = k * layers + l
+    __device__ __forceinline__ void start(uint32_t row, uint32_t blocks, uint32_t layers)
     {
-        k = e / P;
-        j = e - k * P;
-        l = j / T;
-        t = j - l * T;
+        q = row / blocks;
+        tb = row - q * blocks;
+        k = q / layers;
+        l = q - k * layers;
+    }
+    __device__ __forceinline__ void next(uint32_t blocks, uint32_t layers)
+    {
+        if (++tb < blocks) return;
+        tb = 0;
+        ++q;
+        if (++l < layers) return;
+        l = 0;
+        ++k;
     }
 };
 
-// Entry e = k * P + l * T + t of loops that visit e, e + step, e + 2 step, ...:
-// decoded once, then advanced without an integer division per entry.
-struct EntryCursor {
-    EntryIndex x;
-    uint32_t T, layers;
-    __device__ __forceinline__ void start(uint32_t e, uint32_t P, uint32_t T_)
-    {
-        T = T_;
-        layers = P / T_;
-        x.init(e, P, T_);
-    }
-    __device__ __forceinline__ void advance(uint32_t step)
-    {
-        uint32_t t = x.t + step, l = x.l, k = x.k;
-        while (t >= T) {
-            t -= T;
-            if (++l == layers) {
-                l = 0;
-                ++k;
-            }
-        }
-        x.t = t;
-        x.l = l;
-        x.k = k;
-        x.j = t + l * T;
-    }
-};
-
-// LDS for one pass of mixture_prefix: kBlock * kScanPer doubles, one pad
-// slot per kScanPer so a thread's consecutive run is bank-conflict free.
-constexpr int kScanLds = kBlock * kScanPer + kBlock * kScanPer / kScanPer;
-__device__ __forceinline__ int scan_slot(int i) { return i + i / kScanPer; }
-
-// Defensive-mixture proposal and its FP64 inclusive prefix for one sample
-// (one work-group): q_e = (1 - eps) imp_e / I + eps * bv_j / (R * Bsum), with
-// I the work-group sum of the thread partials `local`.  value(x, e) returns
-// imp_e.  Each pass covers kBlock * kScanPer entries: they are computed and
-// stored in coalesced order (entry base + i*kBlock + tid), while the scan
-// runs over kScanPer consecutive entries per thread, transposed through LDS.
-// red holds kBlock/64 + 2 doubles, buf kScanLds doubles of LDS.
 template <class F>
-__device__ __forceinline__ void mixture_prefix(double local, uint32_t n, uint32_t P, uint32_t T, const float* bv,
-                                               double eps, double Bsum, uint32_t R, F value, double* pre,
-                                               double* Qout, double* red, double* buf, uint32_t* bucket)
+__device__ __forceinline__ void mixture_prefix(uint32_t T, uint32_t layers, uint32_t R, const float* bv, double eps,
+                                               double Bsum, F value, double* pre, double* Qout, uint32_t* bucket)
 {
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    double* carry_s = red + kBlock / 64;
-    double* total_s = red + kBlock / 64 + 1;
-    // buckets beyond the total (rounding) keep the last entry
-    if (bucket)
-        for (uint32_t k = (uint32_t)tid; k < kPrefixBuckets; k += (uint32_t)kBlock) bucket[k] = n - 1u;
-    local = wave_sum(local);
-    if (lane == 0) red[wid] = local;
-    __syncthreads();
-    if (tid == 0) {
-        double I = 0.0;
-        for (int i = 0; i < kBlock / 64; ++i) I += red[i];
-        *total_s = I;
-        *carry_s = 0.0;
+    __shared__ double part[2][kPrefixMaxBlock / 64];
+    const uint32_t lane = threadIdx.x & 63u, W = blockDim.x >> 6;
+    const uint32_t wid = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t blocks = (T + 63u) / 64u, rows = R * layers * blocks;
+    const uint32_t row0 = (uint32_t)((uint64_t)rows * wid / W), row1 = (uint32_t)((uint64_t)rows * (wid + 1u) / W);
+    ProposalRow at[kRowsAhead];
+    float imp[kRowsAhead], b[kRowsAhead];
+    bool live[kRowsAhead];
+    // the next rows from `cur` on: their values, zero beyond the run and the layer
+    auto fetch = [&](ProposalRow& cur, uint32_t row) {
+#pragma unroll
+        for (uint32_t u = 0; u < kRowsAhead; ++u) {
+            at[u] = cur;
+            if (row + u + 1u < row1) cur.next(blocks, layers);
+            const uint32_t t = at[u].tb * 64u + lane;
+            live[u] = row + u < row1 && t < T;
+            const uint32_t tc = t < T ? t : T - 1u;
+            const float x = bv[(size_t)at[u].l * T + tc], v = value(at[u], tc, x);
+            b[u] = live[u] ? x : 0.0f;
+            imp[u] = live[u] ? v : 0.0f;
+        }
+    };
+    double si = 0.0, sb = 0.0;
+    ProposalRow cur;
+    cur.start(row0 < rows ? row0 : 0u, blocks, layers);
+    for (uint32_t row = row0; row < row1; row += kRowsAhead) {
+        fetch(cur, row);
+#pragma unroll
+        for (uint32_t u = 0; u < kRowsAhead; ++u) {
+            si += (double)imp[u];
+            sb += (double)b[u];
+        }
+    }
+    si = wave_sum(si);
+    sb = wave_sum(sb);
+    if (lane == 0u) {
+        part[0][wid] = si;
+        part[1][wid] = sb;
     }
     __syncthreads();
-    const double I = *total_s;
+    double I = 0.0;
+    for (uint32_t i = 0; i < W; ++i) I += part[0][i];
     const bool use_imp = I > 0.0 && isfinite(I);
     const double wI = use_imp ? (1.0 - eps) / I : 0.0;
     const double wB = (use_imp ? eps : 1.0) / (Bsum * (double)R);
-    // entries base + i * kBlock + tid: one cursor stepping by kBlock
-    EntryCursor cur;
-    cur.start((uint32_t)tid, P, T);
-    for (uint32_t base = 0; base < n; base += (uint32_t)kBlock * kScanPer) {
-#pragma unroll
-        for (int i = 0; i < kScanPer; ++i) {
-            const uint32_t e = base + (uint32_t)(i * kBlock + tid);
-            double q = 0.0;
-            if (e < n) q = wI * (double)value(cur.x, e) + wB * (double)bv[cur.x.j];
-            buf[scan_slot(i * kBlock + tid)] = q;
-            cur.advance((uint32_t)kBlock);
-        }
-        __syncthreads();
-        double v[kScanPer];
-        double run = 0.0;
-#pragma unroll
-        for (int i = 0; i < kScanPer; ++i) {
-            run += buf[scan_slot(tid * kScanPer + i)];
-            v[i] = run;
-        }
-        const double inc = wave_inclusive_scan(run, lane);
-        double before = __shfl_up(inc, 1, 64);
-        if (lane == 0) before = 0.0;
-        if (lane == 63) red[wid] = inc;
-        __syncthreads();
-        double off = *carry_s;
-        for (int i = 0; i < wid; ++i) off += red[i];
-        const double excl = off + before;
-#pragma unroll
-        for (int i = 0; i < kScanPer; ++i) buf[scan_slot(tid * kScanPer + i)] = excl + v[i];
-        if (bucket) {
-            // entry e takes the buckets k with prefix(e - 1) <= k / B < prefix(e),
-            // i.e. k in [ceil(prefix(e - 1) B), ceil(prefix(e) B)): B is a power of
-            // two, so the products are exact and one ceil per entry suffices
-            const double B = (double)kPrefixBuckets;
-            uint32_t k0 = (uint32_t)fmin(ceil(excl * B), B);
-#pragma unroll
-            for (int i = 0; i < kScanPer; ++i) {
-                const uint32_t e = base + (uint32_t)(tid * kScanPer + i);
-                const uint32_t k1 = (uint32_t)fmin(ceil((excl + v[i]) * B), B);
-                if (e < n)
-                    for (uint32_t k = k0; k < k1; ++k) bucket[k] = e;
-                k0 = k1;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < kScanPer; ++i) {
-            const uint32_t e = base + (uint32_t)(i * kBlock + tid);
-            if (e < n) pre[e] = buf[scan_slot(i * kBlock + tid)];
-        }
-        if (tid == kBlock - 1) *carry_s = off + inc;
-        __syncthreads();
+    // start and end of this wavefront's run, and the total
+    double total = 0.0, carry = 0.0, end = 0.0;
+    for (uint32_t i = 0; i < W; ++i) {
+        if (i == wid) carry = total;
+        total += wI * part[0][i] + wB * part[1][i];
+        if (i == wid) end = total;
     }
-    if (tid == 0) *Qout = *carry_s;
+    // entry e takes the buckets k with prefix(e - 1) <= k / B < prefix(e), i.e.
+    // k in [ceil(prefix(e - 1) B), ceil(prefix(e) B)): B is a power of two, so
+    // the products are exact; buckets beyond the total (rounding) keep the
+    // last entry
+    const double B = (double)kPrefixBuckets;
+    auto first_bucket = [&](double p) { return (uint32_t)fmin(ceil(p * B), B); };
+    if (bucket)
+        for (uint32_t k = first_bucket(total) + threadIdx.x; k < kPrefixBuckets; k += blockDim.x)
+            bucket[k] = R * layers * T - 1u;
+    uint32_t k0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)first_bucket(carry));
+    cur.start(row0 < rows ? row0 : 0u, blocks, layers);
+    for (uint32_t row = row0; row < row1; row += kRowsAhead) {
+        fetch(cur, row);
+        double s[kRowsAhead];
+#pragma unroll
+        for (uint32_t u = 0; u < kRowsAhead; ++u) s[u] = wI * (double)imp[u] + wB * (double)b[u];
+        wave_inclusive_scan(s);
+#pragma unroll
+        for (uint32_t u = 0; u < kRowsAhead; ++u) {
+            if (row + u >= row1) break;
+            const uint32_t t = at[u].tb * 64u + lane;
+            double p = carry + s[u];
+            p = p < end ? p : end;
+            if (row + u + 1u == row1 && (t + 1u >= T || lane == 63u)) p = end;
+            const size_t base = (size_t)at[u].q * T;
+            if (live[u]) pre[base + t] = p;
+            if (bucket) {
+                const uint32_t k1 = first_bucket(p);
+                const uint32_t last = (uint32_t)__builtin_amdgcn_readlane((int)k1, 63);
+                if (last != k0) {
+                    uint32_t k = (uint32_t)__shfl_up((int)k1, 1u, 64);
+                    if (lane == 0u) k = k0;
+                    if (live[u])
+                        for (; k < k1; ++k) bucket[k] = (uint32_t)base + t;
+                    k0 = last;
+                }
+            }
+            carry += wave_last(s[u]);
+        }
+    }
+    if (threadIdx.x == 0) *Qout = total;
+}
+
+// Threads of a work-group of mixture_prefix: the runs of a wavefront should be
+// long, but few samples have to fill the chip by themselves.  Measured (us per
+// launch, 256 / 512 / 1024 threads): many samples of 91,000 entries and more
+// 2264 / 2180 / 2579 and 4363 / 3346 / 3684, 80 samples 380 / 214 / 144; many
+// samples of 2,000 entries (37 rows) 48 / 83 / 155, 121 of them 16 / 12 / 11.
+inline uint32_t prefix_block(const MeshDev& m, uint32_t R, uint32_t slots, int cus)
+{
+    if (slots <= 2u * (uint32_t)std::max(1, cus)) return 1024u;
+    const uint64_t rows = (uint64_t)R * m.layers * ((m.T + 63u) / 64u);
+    return rows < 256u ? 256u : 512u;
 }
 
 struct ImportanceParams {
@@ -383,31 +396,22 @@ __global__ void __launch_bounds__(kBlock) hase_column_list_kernel(PathParams q)
 // beta * V proposal shared by every sample (one work-group): the mixture with
 // no importance term, q_e = bv_j / (R * Bsum), its FP64 prefix, total and
 // buckets in slot 0 of the prefix tables.
-__global__ void __launch_bounds__(kBlock) hase_beta_volume_prefix_kernel(ImportanceParams p)
+__global__ void __launch_bounds__(kPrefixMaxBlock) hase_beta_volume_prefix_kernel(ImportanceParams p)
 {
-    const MeshDev& m = p.m;
-    const uint32_t T = m.T, P = T * m.layers;
-    __shared__ double red[kBlock / 64 + 2];
-    __shared__ double buf[kScanLds];
-    mixture_prefix(0.0, p.R * P, P, T, m.bv, p.eps, p.Bsum, p.R, [&](const EntryIndex&, uint32_t) { return 0.0f; },
-                   p.prefix, p.Q, red, buf, p.buckets);
+    mixture_prefix(p.m.T, p.m.layers, p.R, p.m.bv, p.eps, p.Bsum,
+                   [&](const ProposalRow&, uint32_t, float) { return 0.0f; }, p.prefix, p.Q, p.buckets);
 }
 
 // Mixture prefix of the importance maps, one work-group per sample.
-__global__ void __launch_bounds__(kBlock) hase_prefix_kernel(ImportanceParams p)
+__global__ void __launch_bounds__(kPrefixMaxBlock) hase_prefix_kernel(ImportanceParams p)
 {
     const uint32_t slot = p.active ? p.active[blockIdx.x] : blockIdx.x;
     if (slot >= p.slots) return;
-    const MeshDev& m = p.m;
-    const uint32_t T = m.T, P = T * m.layers;
-    const uint32_t n = p.R * P;
+    const uint32_t T = p.m.T, n = p.R * p.m.layers * T;
     const float* imp = p.imp + (size_t)slot * n;
-    __shared__ double red[kBlock / 64 + 2];
-    __shared__ double buf[kScanLds];
-    double local = 0.0;
-    for (uint32_t e = threadIdx.x; e < n; e += kBlock) local += (double)imp[e];
-    mixture_prefix(local, n, P, T, m.bv, p.eps, p.Bsum, p.R, [&](const EntryIndex&, uint32_t e) { return imp[e]; },
-                   p.prefix + (size_t)slot * n, p.Q + slot, red, buf,
+    mixture_prefix(T, p.m.layers, p.R, p.m.bv, p.eps, p.Bsum,
+                   [&](const ProposalRow& r, uint32_t t, float) { return imp[(size_t)r.q * T + t]; },
+                   p.prefix + (size_t)slot * n, p.Q + slot,
                    p.buckets ? p.buckets + (size_t)slot * kPrefixBuckets : nullptr);
 }
 
@@ -430,62 +434,30 @@ struct LearnedParams {
     uint32_t* buckets = nullptr;   // [slots * kPrefixBuckets] or null
 };
 
-// An entry's slice and layer change only every T entries of a thread's
-// ascending run, so the slice's image plane, the layer's row of cluster
-// logits and the height difference are kept per thread and recomputed on a
-// change; per entry remain the cluster column, the logit, the centroid and
-// beta * V.  The reciprocal is the hardware one (1 ulp).
-struct LearnedRow {
-    uint32_t k = ~0u, l = ~0u;
-    float zi = 0.0f, dz = 0.0f;
-    const float* row = nullptr;
-};
-
-__device__ __forceinline__ float learned_importance(const LearnedParams& p, const SampleGeom& sp, const float* lg,
-                                                    const EntryIndex& x, LearnedRow& r)
-{
-    const MeshDev& m = p.m;
-    if (x.k != r.k) {
-        r.k = x.k;
-        r.zi = (float)image_plane(sp.plane, (int)m.layers, (x.k + 1u) >> 1, x.k & 1u);
-        r.l = ~0u;
-    }
-    if (x.l != r.l) {
-        r.l = x.l;
-        r.row = lg + (size_t)x.k * p.C + p.cl_lev[x.l];
-        r.dz = ((float)x.l + 0.5f - r.zi) * m.h;
-    }
-    const float y = fminf(r.row[p.cl_tri[x.t]], 80.0f);
-    const float2 cxy = p.centroid[x.t];
-    const float dx = cxy.x - sp.px, dy = cxy.y - sp.py;
-    const float d2 = fmaf(dx, dx, fmaf(dy, dy, r.dz * r.dz));
-    const float v = m.bv[x.j] * __expf(y) * __builtin_amdgcn_rcpf(4.0f * kPi * d2);
-    return (v >= 0.0f && !isinf(v)) ? v : 0.0f;
-}
-
-__global__ void __launch_bounds__(kBlock) hase_learned_importance_kernel(LearnedParams p)
+// The slice's image plane, the layer's row of cluster logits and the height
+// difference are uniform in a row; per entry remain the cluster column, the
+// logit, the centroid and beta * V.  The reciprocal is the hardware one (1 ulp).
+__global__ void __launch_bounds__(kPrefixMaxBlock) hase_learned_importance_kernel(LearnedParams p)
 {
     const uint32_t slot = blockIdx.x;
     if (slot >= p.slots) return;
     const MeshDev& m = p.m;
-    const uint32_t T = m.T, P = T * m.layers;
-    const uint32_t n = p.R * P;
+    const uint32_t n = p.R * m.layers * m.T;
     const SampleGeom sp = sample_point(p.pts, m.np, p.sample_base + slot);
     const float* lg = p.logits + (size_t)slot * p.R * p.C;
-    LearnedRow row;
-    auto value = [&](const EntryIndex& x, uint32_t) { return learned_importance(p, sp, lg, x, row); };
-    __shared__ double red[kBlock / 64 + 2];
-    __shared__ double buf[kScanLds];
-    double local = 0.0;
-    EntryCursor cur;
-    cur.start(threadIdx.x, P, T);
-    for (uint32_t e = threadIdx.x; e < n; e += kBlock) {
-        local += (double)value(cur.x, e);
-        cur.advance((uint32_t)kBlock);
-    }
-    row = LearnedRow{};
-    mixture_prefix(local, n, P, T, m.bv, p.eps, p.Bsum, p.R, value, p.prefix + (size_t)slot * n, p.Q + slot, red,
-                   buf, p.buckets ? p.buckets + (size_t)slot * kPrefixBuckets : nullptr);
+    auto value = [&](const ProposalRow& r, uint32_t t, float bv) {
+        const float* row = lg + (size_t)r.k * p.C + ((ConstU32*)p.cl_lev)[r.l];
+        const float zi = (float)image_plane(sp.plane, (int)m.layers, (r.k + 1u) >> 1, r.k & 1u);
+        const float dz = ((float)r.l + 0.5f - zi) * m.h;
+        const float y = fminf(row[p.cl_tri[t]], 80.0f);
+        const float2 cxy = p.centroid[t];
+        const float dx = cxy.x - sp.px, dy = cxy.y - sp.py;
+        const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+        const float v = bv * __expf(y) * __builtin_amdgcn_rcpf(4.0f * kPi * d2);
+        return (v >= 0.0f && !isinf(v)) ? v : 0.0f;
+    };
+    mixture_prefix(m.T, m.layers, p.R, m.bv, p.eps, p.Bsum, value, p.prefix + (size_t)slot * n, p.Q + slot,
+                   p.buckets ? p.buckets + (size_t)slot * kPrefixBuckets : nullptr);
 }
 
 struct TraceParams {
@@ -1237,7 +1209,8 @@ void launch_importance(hase_context* ctx, ImportanceParams& ip, uint32_t slots)
     hipLaunchKernelGGL(hase_column_list_kernel, list, dim3(kBlock), 0, ctx->stream, q);
     HIP_CHECK(hipGetLastError());
     if (!ip.transfer) {
-        hipLaunchKernelGGL(hase_prefix_kernel, dim3(slots), dim3(kBlock), 0, ctx->stream, ip);
+        const uint32_t threads = prefix_block(ip.m, ip.R, slots, cus);
+        hipLaunchKernelGGL(hase_prefix_kernel, dim3(slots), dim3(threads), 0, ctx->stream, ip);
         HIP_CHECK(hipGetLastError());
     }
 }
@@ -1256,7 +1229,7 @@ void build_shared_prefix(hase_context* ctx, BatchTimers& tm)
     ip.Q = ctx->Q.p;
     ip.buckets = ctx->buckets.p;
     hipEvent_t i0 = record(ctx);
-    hipLaunchKernelGGL(hase_beta_volume_prefix_kernel, dim3(1), dim3(kBlock), 0, ctx->stream, ip);
+    hipLaunchKernelGGL(hase_beta_volume_prefix_kernel, dim3(1), dim3(kPrefixMaxBlock), 0, ctx->stream, ip);
     HIP_CHECK(hipGetLastError());
     tm.imp.emplace_back(i0, record(ctx));
     ctx->stats.importance_launches++;
@@ -1295,7 +1268,10 @@ void build_proposal(hase_context* ctx, uint32_t b0, const uint32_t* sample_of, u
         lp.prefix = ctx->prefix.p;
         lp.Q = ctx->Q.p;
         lp.buckets = ctx->buckets.p;
-        hipLaunchKernelGGL(hase_learned_importance_kernel, dim3(slots), dim3(kBlock), 0, ctx->stream, lp);
+        int cus = 0;
+        HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+        const uint32_t threads = prefix_block(m, R, slots, cus);
+        hipLaunchKernelGGL(hase_learned_importance_kernel, dim3(slots), dim3(threads), 0, ctx->stream, lp);
         HIP_CHECK(hipGetLastError());
         tm.inf.emplace_back(a0, a1);
         tm.prop.emplace_back(a1, record(ctx));

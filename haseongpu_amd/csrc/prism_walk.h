@@ -949,10 +949,8 @@ HASE_HD inline WalkOut walk_edges(const MeshDev& m, float ax, float ay, float za
 // the image lies exactly on a plane of the unfolded axis.
 HASE_HD inline int image_plane(int lv, int layers, uint32_t nrefl, uint32_t first)
 {
-    int mr = (int)nrefl;
-    if (nrefl == 0) return lv;
-    if (first == 1u) return (nrefl & 1u) ? mr * layers + (layers - lv) : mr * layers + lv;
-    return (nrefl & 1u) ? -(mr - 1) * layers - lv : -mr * layers + lv;
+    const int n = (int)nrefl, odd = n & 1;
+    return ((first == 1u ? n : -n) + odd) * layers + (odd ? -lv : lv);
 }
 
 constexpr float kLog2e = 1.44269504088896341f;

@@ -223,9 +223,6 @@ __device__ __forceinline__ void start_ray(const MeshDev& m, const ItemCtx& c, ui
 // table is constant for the launch and the address uniform in the wavefront)
 // and with their pointers known to be global, so that they cost the walks no
 // vector registers and no generic-address loads.
-// written by earlier kernels only, indexed uniformly: read through the scalar cache
-typedef const __attribute__((address_space(4))) uint32_t ConstU32;
-
 template <class T>
 __device__ __forceinline__ void as_global(T*& p)
 {
