@@ -8,12 +8,12 @@
 //             list of slots with work and the exclusive prefix of their queue
 //             items (rays_per_item rays each);
 //   trace     (persistent grid): each wavefront takes queue_chunk items at a
-//             time from a device cursor; its lanes walk the item's rays and,
-//             whenever refill_lanes of them are idle, start the next rays of
-//             the item, so a long ray no longer holds 63 finished lanes; the
+//             time from a device cursor; its lanes walk the item's rays, 256
+//             at a time sorted by estimated length, or with refill_lanes start
+//             the next rays of the item whenever that many lanes are idle; the
 //             wavefront's FP64 sums are written per item (no atomics);
-//   finalize  (one lane per listed slot): pools its items in order, forms
-//             phiAse / mse in FP64 and decides convergence.
+//   finalize  (one wavefront per listed slot): pools its items, forms phiAse /
+//             mse in FP64 and decides convergence.
 // All round inputs live in device memory, so the rounds of a batch replay one
 // captured hipGraph back to back; rounds with nothing left to do are empty.
 // Slots of several problems (meshes with their own proposal, spectra and
@@ -431,20 +431,27 @@ __global__ void __launch_bounds__(kQueueMaxBlock) hase_queue_trace_kernel(QueueS
     block_count(steps, red[1], &q.counters[1]);
 }
 
+// A wavefront per listed slot: its lanes read the items' sums side by side
+// (one lane reading 200 of them in turn took 83 us a round for 1,210 samples,
+// 6 so).
 __global__ void hase_queue_finalize_kernel(QueueState q)
 {
-    const uint32_t a = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t a = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63u;
     if (a >= q.scalars[kNActive]) return;
     const uint32_t slot = q.list[a];
     const ProblemDev& pd = q.problems[q.slot_problem[slot]];
-    double a1 = q.s1[slot], a2 = q.s2[slot];
-    uint32_t drop = q.dropped[slot];
-    for (uint32_t it = q.item_off[a]; it < q.item_off[a + 1]; ++it) {
+    double a1 = 0.0, a2 = 0.0;
+    uint32_t drop = 0;
+    for (uint32_t it = q.item_off[a] + lane; it < q.item_off[a + 1]; it += 64u) {
         const double2 v = q.partial[it];
         a1 += v.x;
         a2 += v.y;
         drop += q.partial_drop[it];
     }
+    a1 = q.s1[slot] + wave_sum(a1);
+    a2 = q.s2[slot] + wave_sum(a2);
+    drop = q.dropped[slot] + (uint32_t)wave_sum_u64((unsigned long long)drop);
+    if (lane != 0u) return;
     const uint32_t N = q.N[slot] + q.nrays[slot];
     q.s1[slot] = a1;
     q.s2[slot] = a2;
@@ -623,7 +630,7 @@ float queue_run(hipStream_t stream, int device, const hase_tuning_t& tu, const Q
     std::memset(&one, 0, sizeof(one));
     if (single) one = *single;
     const int grid = std::max(1, cus) * std::max(1, per);
-    const uint32_t fin_blocks = std::max(1u, (slots + 255u) / 256u);
+    const uint32_t fin_blocks = std::max(1u, (slots + 3u) / 4u);   // a wavefront per slot
     // allocation-free calls (an arena installed) create no events and report no time
     const bool timed = g_arena == nullptr;
     hipEvent_t t0 = nullptr, t1 = nullptr;
