@@ -42,6 +42,7 @@ struct hase_context {
     hase::DevBuf<float2> pts;
     hase::DevBuf<float> beta, beta_col, bv, refl, c1, c2;
     hase::DevBuf<float> imp;
+    hase::DevBuf<float> map_out;       // maps in the caller's order, on their way to the host
     uint32_t path_cap = 32;            // triangles of an importance path that the map kernel stores
     uint64_t path_tiles = 0;           // tiles of 64 paths that the storage holds
     hase::DevBuf<uint2> path;          // triangles and exit sigmas of a sub-batch of paths
