@@ -65,66 +65,112 @@ struct GemmArgs {
 
 enum { EPI_NONE = 0, EPI_BIAS_SILU = 1, EPI_GATE = 2, EPI_BIAS = 3 };
 
-constexpr int kTM = 64, kTN = 64, kTK = 16;
+// Tiles of 32 x 128 (the network's width, so A is read once), four wavefronts
+// of 32 x 32 each through v_mfma_f32_32x32x2_f32: FP32 operands and sums.  32
+// steps of K are staged in LDS while the next 32 are on their way to
+// registers, by 16-byte loads along whichever index is contiguous.  A product
+// of 16,384 x 128 by 128 x 128 has 0.54 GFLOP and 17 MB to read and write, 4
+// us of either; it took 35 us with 4-byte loads, one element at a time, and
+// scalar FMAs on 64 x 64 tiles, and takes 17 (tiles of 64 rows 21: one
+// work-group per CU has nothing to run beside its loads).
+constexpr int kTM = 32, kTN = 128, kTK = 32;
+constexpr int kChunk = 16;   // split-K chunks are multiples of this
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// kTK x kRows elements (row r0 + r, step k) of a matrix with strides sr and
+// sk, zero beyond rows and ke, as float4 per thread: along k if that is
+// contiguous, else along the rows.
+template <int kRows>
+struct TileLoad {
+    static constexpr int kPer = kTK * kRows / 4 / 256;
+    float4 v[kPer];
+    __device__ __forceinline__ void fetch(const float* m, long long sr, long long sk, int r0, int rows, int k0, int ke,
+                                          int tid)
+    {
+        const bool along_k = sk == 1;
+        const bool wide = (along_k ? sr % 4 == 0 : sr == 1 && sk % 4 == 0) && (reinterpret_cast<uintptr_t>(m) & 15u) == 0u;
+#pragma unroll
+        for (int s = 0; s < kPer; ++s) {
+            const int e = tid + 256 * s;
+            const int r = r0 + (along_k ? e / (kTK / 4) : 4 * (e % (kRows / 4)));
+            const int k = k0 + (along_k ? 4 * (e % (kTK / 4)) : e / (kRows / 4));
+            const int left = along_k ? (r < rows ? ke - k : 0) : (k < ke ? rows - r : 0);   // elements in range
+            const float* at = m + (long long)r * sr + (long long)k * sk;
+            const long long step = along_k ? sk : sr;
+            if (wide && left >= 4) {
+                v[s] = *reinterpret_cast<const float4*>(at);
+            } else {
+                v[s].x = left > 0 ? at[0] : 0.0f;
+                v[s].y = left > 1 ? at[step] : 0.0f;
+                v[s].z = left > 2 ? at[2 * step] : 0.0f;
+                v[s].w = left > 3 ? at[3 * step] : 0.0f;
+            }
+        }
+    }
+    __device__ __forceinline__ void put(float (*t)[kRows + 4], bool along_k, int tid) const
+    {
+#pragma unroll
+        for (int s = 0; s < kPer; ++s) {
+            const int e = tid + 256 * s;
+            if (along_k) {
+                const int r = e / (kTK / 4), k = 4 * (e % (kTK / 4));
+                t[k][r] = v[s].x;
+                t[k + 1][r] = v[s].y;
+                t[k + 2][r] = v[s].z;
+                t[k + 3][r] = v[s].w;
+            } else {
+                *reinterpret_cast<float4*>(&t[e / (kRows / 4)][4 * (e % (kRows / 4))]) = v[s];
+            }
+        }
+    }
+};
 
 __global__ void __launch_bounds__(256) gemm_kernel(GemmArgs g)
 {
-    __shared__ float As[kTK][kTM + 4];
-    __shared__ float Bs[kTK][kTN + 4];
-    const int tid = threadIdx.x;
-    const int tx = tid & 15, ty = tid >> 4;
+    __shared__ __attribute__((aligned(16))) float As[kTK][kTM + 4];
+    __shared__ __attribute__((aligned(16))) float Bs[kTK][kTN + 4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int i0 = blockIdx.y * kTM, j0 = blockIdx.x * kTN;
     const int kb = blockIdx.z * g.kchunk;
     const int ke = min(g.K, kb + g.kchunk);
-    float acc[4][4];
+    const int jw = 32 * wave;   // the wavefront's columns of the tile
+    const int half = lane >> 5, col = lane & 31;
+    f32x16 acc;
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[r][c] = 0.0f;
+    for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+    TileLoad<kTM> a;
+    TileLoad<kTN> b;
+    a.fetch(g.A, g.sai, g.sak, i0, g.M, kb, ke, tid);
+    b.fetch(g.B, g.sbj, g.sbk, j0, g.N, kb, ke, tid);
     for (int k0 = kb; k0 < ke; k0 += kTK) {
-        for (int e = tid; e < kTK * kTM; e += 256) {
-            int kk, ii;
-            if (g.sak == 1) { kk = e % kTK; ii = e / kTK; } else { ii = e % kTM; kk = e / kTM; }
-            const int i = i0 + ii, k = k0 + kk;
-            As[kk][ii] = (i < g.M && k < ke) ? g.A[(long long)i * g.sai + (long long)k * g.sak] : 0.0f;
-        }
-        for (int e = tid; e < kTK * kTN; e += 256) {
-            int kk, jj;
-            if (g.sbj == 1) { jj = e % kTN; kk = e / kTN; } else { kk = e % kTK; jj = e / kTK; }
-            const int j = j0 + jj, k = k0 + kk;
-            Bs[kk][jj] = (j < g.N && k < ke) ? g.B[(long long)k * g.sbk + (long long)j * g.sbj] : 0.0f;
-        }
+        a.put(As, g.sak == 1, tid);
+        b.put(Bs, g.sbk == 1, tid);
         __syncthreads();
+        if (k0 + kTK < ke) {
+            a.fetch(g.A, g.sai, g.sak, i0, g.M, k0 + kTK, ke, tid);
+            b.fetch(g.B, g.sbj, g.sbk, j0, g.N, k0 + kTK, ke, tid);
+        }
 #pragma unroll
-        for (int kk = 0; kk < kTK; ++kk) {
-            float a[4], b[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) a[r] = As[kk][ty * 4 + r];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) b[c] = Bs[kk][tx * 4 + c];
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) acc[r][c] = fmaf(a[r], b[c], acc[r][c]);
+        for (int kk = 0; kk < kTK; kk += 2) {
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(As[kk + half][col], Bs[kk + half][jw + col], acc, 0, 0, 0);
         }
         __syncthreads();
     }
     float* C = g.C + (long long)blockIdx.z * g.split_stride;
+    const int j = j0 + jw + col;
+    if (j >= g.N) return;
+    const float bias = g.epi == EPI_BIAS || g.epi == EPI_BIAS_SILU ? g.bias[j] : 0.0f;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int i = i0 + ty * 4 + r;
+    for (int r = 0; r < 16; ++r) {
+        const int i = i0 + (r & 3) + 4 * half + 8 * (r >> 2);
         if (i >= g.M) continue;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int j = j0 + tx * 4 + c;
-            if (j >= g.N) continue;
-            const long long at = (long long)i * g.ldc + j;
-            float v = acc[r][c];
-            if (g.epi == EPI_BIAS || g.epi == EPI_BIAS_SILU) v += g.bias[j];
-            if (g.epi == EPI_GATE) v *= silu_grad(g.gate[at]);
-            C[at] = v;
-            if (g.epi == EPI_BIAS_SILU) g.act[at] = silu_exact(v);
-        }
+        const long long at = (long long)i * g.ldc + j;
+        float v = acc[r];
+        if (g.epi == EPI_BIAS || g.epi == EPI_BIAS_SILU) v += bias;
+        if (g.epi == EPI_GATE) v *= silu_grad(g.gate[at]);
+        C[at] = v;
+        if (g.epi == EPI_BIAS_SILU) g.act[at] = silu_exact(v);
     }
 }
 
@@ -134,7 +180,8 @@ __global__ void split_sum_kernel(const float* part, int splits, long long stride
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= count) return;
     float s = 0.0f;
-    for (int z = 0; z < splits; ++z) s += part[(long long)z * stride + i];
+#pragma unroll 8
+    for (int z = 0; z < splits; ++z) s += part[(long long)z * stride + i];   // eight loads in flight
     out[i] = s;
 }
 
@@ -242,7 +289,7 @@ struct Trainer {
         const int n = g.K;
         const int sp = std::max(1, std::min(splits, (n + 255) / 256));
         int chunk = (n + sp - 1) / sp;
-        chunk = (chunk + kTK - 1) / kTK * kTK;
+        chunk = (chunk + kChunk - 1) / kChunk * kChunk;
         const int used = (n + chunk - 1) / chunk;
         g.C = part.p;
         g.ldc = g.N;
@@ -373,7 +420,6 @@ void use_device(int32_t device)
 
 // ------------------------------------------------------------ BF16 inference
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kInferBlock = 1024;
 constexpr int kInferWaves = kInferBlock / 64;
