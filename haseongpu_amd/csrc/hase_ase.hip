@@ -382,8 +382,11 @@ __global__ void __launch_bounds__(kBlock) hase_column_list_kernel(PathParams q)
         int lv0, nlev;
         ci.decode((uint32_t)(it - a * per), unused, k, lv0, nlev);
         float v[kLevelGroup];
-        steps += column_entries(m, GlobalTriangles{}, p.c1, p.c2, p.n_lambda, p.inv_lambda, t0, lv0, nlev, k, sp.px,
-                                sp.py, sp.plane, p.transfer != 0, v);
+        auto walk = [&](const auto& fetch) {
+            return column_entries(m, fetch, p.c1, p.c2, p.n_lambda, p.inv_lambda, t0, lv0, nlev, k, sp.px, sp.py,
+                                  sp.plane, p.transfer != 0, v);
+        };
+        steps += m.edges ? walk(GlobalEdges{}) : walk(GlobalTriangles{});
         float* imp = p.imp + ((size_t)slot * p.R + k) * P + t0;
 #pragma unroll
         for (int g = 0; g < kLevelGroup; ++g)
@@ -963,16 +966,24 @@ std::unique_ptr<hase_context> create_context(const hase_mesh_t* mesh, const hase
         const double most = 16.0 + 1.9 * std::sqrt((double)T / area) * 2.0 * std::sqrt(r2);
         ctx->path_cap = (uint32_t)std::min(10000.0, std::max(32.0, std::ceil(most / 16.0) * 16.0));
     }
-    ctx->rec.upload(rec.data(), rec.size(), ctx->stream);
+    // one form of the records in allocation-free calls: 64 B per triangle below
+    // 2^19, 48 from there
+    const bool with_edges = !g_arena || T < (1u << 19);
+    if (!g_arena || !with_edges) ctx->rec.upload(rec.data(), rec.size(), ctx->stream);
     ctx->user2dev_dev.upload(ctx->user2dev.data(), T, ctx->stream);
     std::vector<float2>& pts = ctx->pts_host;
     pts.resize(np);
     for (uint32_t i = 0; i < np; ++i) pts[i] = make_float2((float)px[i], (float)py[i]);
     {
         const EdgeRecords er = edge_records(rec.data(), T, pts.data(), np);
-        ctx->edges.upload(er.global.data(), er.global.size(), ctx->stream);
-        if (er.kind) ctx->lds_rec.upload(er.staged.data(), er.staged.size(), ctx->stream);
-        ctx->lds_kind = er.kind;
+        if (with_edges) ctx->edges.upload(er.global.data(), er.global.size(), ctx->stream);
+        // an allocation-free call stages where its scratch has room to spare
+        const size_t slices = e->use_reflections ? 1u + 2u * (size_t)std::max(1u, e->max_reflections) : 1u;
+        const size_t one_sample = slices * ctx->P * 12u;
+        if (er.kind && (!g_arena || g_arena->remaining() / 4u > one_sample)) {
+            ctx->lds_rec.upload(er.staged.data(), er.staged.size(), ctx->stream);
+            ctx->lds_kind = er.kind;
+        }
         HIP_CHECK(hipStreamSynchronize(ctx->stream));
     }
     ctx->tuning.stage_lds = 1u;
@@ -1120,7 +1131,7 @@ uint32_t reserve_batch(hase_context* ctx, uint32_t want, size_t budget = 0, bool
         const size_t keep = ((size_t)64 << 10) + (shared ? tables_b : 0u);
         // importance paths and their list, where several slots fit beside
         // them (the map's columns are walked level group by level group else)
-        if (!shared && ctx->path_tiles == 0 && g_arena->remaining() / 8u > per_slot + keep)
+        if (!shared && ctx->edges.p && ctx->path_tiles == 0 && g_arena->remaining() / 8u > per_slot + keep)
             reserve_paths(ctx, (uint64_t)1 << 32, 0);
         if (ctx->path_tiles) per_slot += ctx->T * sizeof(uint32_t);
         size_t left = g_arena->remaining();
@@ -1198,7 +1209,7 @@ void launch_importance(hase_context* ctx, ImportanceParams& ip, uint32_t slots)
     q.p = ip;
     q.rows = std::min(ctx->path_cap, kPathEntries - 1u) + 1u;
     // the list numbers paths in 32 bits
-    const uint64_t held = (uint64_t)slots * T <= 0xFFFFFFFFull ? reserve_paths(ctx, tiles, (size_t)slots * T) : 0u;
+    const uint64_t held = ip.m.edges && (uint64_t)slots * T <= 0xFFFFFFFFull ? reserve_paths(ctx, tiles, (size_t)slots * T) : 0u;
     if (held) {
         HIP_CHECK(hipMemsetAsync(ctx->path_count.p, 0, sizeof(uint32_t), ctx->stream));
         q.path = ctx->path.p;

@@ -62,7 +62,10 @@ constexpr uint32_t kLdsCompact = 1u, kLdsIndexed = 2u;
 //                 cladding << 15, u16 [3T] point index of vertex k: 12 B per
 //                 triangle and 8 B per point, up to ~10,100 triangles; a step
 //                 picks the two links and the vertex by f (~8 instructions more)
-constexpr uint32_t kLdsEdges = 4u, kLdsIndexedEdges = 5u, kLdsTwins = 6u;
+// Contexts that hold no edge records (allocation-free calls on meshes of 2^19
+// triangles and more, where they would take 16 B per triangle more of the
+// fixed scratch than the 48-byte ones) walk those: kRecords.
+constexpr uint32_t kLdsEdges = 4u, kLdsIndexedEdges = 5u, kLdsTwins = 6u, kRecords = 7u;
 
 // Unsigned division by a divisor fixed per mesh, exact for every n (Granlund
 // and Montgomery, "Division by invariant integers using multiplication", PLDI
@@ -382,6 +385,15 @@ struct GlobalEdges {
         n = make_float2(bits_to_float(q.x), bits_to_float(q.y));
         l = make_uint2(q.z, q.w);
     }
+    // links behind edges e1 and e2 of t as the column walks take them
+    HASE_HD void words(const MeshDev& m, uint32_t t, uint32_t e1, uint32_t e2, uint32_t& w1, uint32_t& w2,
+                       uint32_t& own) const
+    {
+        w1 = out(m, t, e1, own);
+        w2 = out(m, t, e2, own);
+    }
+    HASE_HD static uint32_t next(uint32_t w) { return w >> 6; }
+    HASE_HD static uint32_t edge(uint32_t w) { return (w >> 4) & 3u; }
 };
 
 // Links of the LDS formats: 15-bit record numbers 3 t + f.
@@ -475,7 +487,8 @@ struct LdsTwins : ShortLinks {
 template <uint32_t kKind>
 using EdgeFetch = std::conditional_t<kKind == kLdsEdges, LdsEdges,
                                      std::conditional_t<kKind == kLdsIndexedEdges, LdsIndexedEdges,
-                                                        std::conditional_t<kKind == kLdsTwins, LdsTwins, GlobalEdges>>>;
+                                                        std::conditional_t<kKind == kLdsTwins, LdsTwins,
+                                                                           std::conditional_t<kKind == kRecords, GlobalTriangles, GlobalEdges>>>>;
 
 template <uint32_t kKind>
 HASE_HD inline EdgeFetch<kKind> edge_fetch(const uint4* s, uint32_t T, uint32_t np)
@@ -489,6 +502,8 @@ HASE_HD inline EdgeFetch<kKind> edge_fetch(const uint4* s, uint32_t T, uint32_t 
     } else if constexpr (kKind == kLdsTwins) {
         const uint16_t* twin = reinterpret_cast<const uint16_t*>(xy + np);
         return LdsTwins{{}, xy, twin, twin + 3u * T};
+    } else if constexpr (kKind == kRecords) {
+        return GlobalTriangles{};
     } else {
         return GlobalEdges{};
     }
@@ -941,6 +956,13 @@ HASE_HD inline WalkOut walk_edges(const MeshDev& m, float ax, float ay, float za
     o.gain_len = (sig - clad_sig) * D;
     o.clad_len = clad_sig * D;
     return o;
+}
+
+HASE_HD inline WalkOut walk_edges(const MeshDev& m, float ax, float ay, float za, uint32_t t, uint32_t layer, float2 p0,
+                                  float2 p1, float2 p2, float ex, float ey, float ze, uint32_t nrefl, uint32_t first,
+                                  const GlobalTriangles& records)
+{
+    return walk_ray(m, ax, ay, za, t, layer, p0, p1, p2, ex, ey, ze, nrefl, first, records);
 }
 
 // Height, in layer units, of the mirror image of a sample point on plane

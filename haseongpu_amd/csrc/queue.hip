@@ -259,15 +259,15 @@ __device__ __forceinline__ ProblemDev table_problem(const ProblemDev* at)
 // they sit in scalar registers.  kKind (single problem whose edge records fit
 // in LDS: kLdsEdges, kLdsIndexedEdges or kLdsTwins): the work-group first
 // copies them into LDS and the walks read them there; beta stays in global
-// memory.  0: the walks read the item's problem's records from global memory
-// (the lane-refill variant the 48-byte ones).
+// memory.  0: the walks read the item's problem's edge records from global
+// memory (the lane-refill variant the 48-byte ones, as does kRecords).
 template <bool kRefill, bool kTable, uint32_t kKind>
 __global__ void __launch_bounds__(kQueueMaxBlock) hase_queue_trace_kernel(QueueState q, ProblemDev one)
 {
     const uint32_t n_active = q.scalars[kNActive];
     if (n_active == 0u) return;
     const uint4* staged = nullptr;
-    if constexpr (kKind != 0u) {
+    if constexpr (kKind != 0u && kKind != kRecords) {
         __shared__ uint4 s_tri[kLdsStageWords];
         const uint32_t n = one.m.lds_words;
         for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) s_tri[i] = one.m.lds_rec[i];
@@ -620,7 +620,8 @@ float queue_run(hipStream_t stream, int device, const hase_tuning_t& tu, const Q
     const bool table = single == nullptr;
     // LDS staging: single problem, no lane refill, mesh small enough
     const uint32_t lds = tu.stage_lds && !table && !refill && single->m.lds_rec != nullptr ? single->m.lds_kind : 0u;
-    auto kernel = lds == kLdsEdges ? hase_queue_trace_kernel<false, false, kLdsEdges>
+    auto kernel = single && !single->m.edges && !refill ? hase_queue_trace_kernel<false, false, kRecords>
+                : lds == kLdsEdges ? hase_queue_trace_kernel<false, false, kLdsEdges>
                 : lds == kLdsIndexedEdges ? hase_queue_trace_kernel<false, false, kLdsIndexedEdges>
                 : lds == kLdsTwins ? hase_queue_trace_kernel<false, false, kLdsTwins>
                 : refill ? (table ? hase_queue_trace_kernel<true, true, 0u> : hase_queue_trace_kernel<true, false, 0u>)

@@ -60,7 +60,7 @@ def test_replay_equals_the_column_walks(lib, name, cap, transfer):
         p, lv = int(s) % Np, int(s) // Np
         replay, columns = np.full(R * T * (L - 1), -1.0, np.float32), np.zeros(R * T * (L - 1), np.float32)
         n1, n2, full = U64(0), U64(0), U32(0)
-        lib.column_path_host(U32(T), U32(L - 1), F32(h), ptr(rec, U32), ptr(pts, F32), U32(Np), ptr(beta, F32), ptr(bv, F32), ptr(refl, F32),
+        assert 0 == lib.column_path_host(U32(T), U32(L - 1), F32(h), ptr(rec, U32), ptr(pts, F32), U32(Np), ptr(beta, F32), ptr(bv, F32), ptr(refl, F32),
                              ptr(ni, F32), F32(float(med.value("claddingAbsorption"))), ptr(c1, F32), ptr(c2, F32),
                              U32(len(c1)), F32(pts[p, 0]), F32(pts[p, 1]), C.c_int(lv), U32(R), C.c_int(transfer),
                              U32(cap), ptr(replay, F32), ptr(columns, F32), C.byref(n1), C.byref(n2), C.byref(full))

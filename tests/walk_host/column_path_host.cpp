@@ -46,6 +46,11 @@ extern "C" int column_path_host(uint32_t T, uint32_t layers, float h, const uint
         float v[kLevelGroup];
         *column_steps += column_entries(m, fetch, c1, c2, n_lambda, 1.0f / (float)n_lambda, t0, lv0, nlev, k, px, py,
                                         plane, transfer != 0, v);
+        float u[kLevelGroup];
+        column_entries(m, GlobalEdges{}, c1, c2, n_lambda, 1.0f / (float)n_lambda, t0, lv0, nlev, k, px, py, plane,
+                       transfer != 0, u);
+        for (int g = 0; g < nlev; ++g)
+            if (u[g] != v[g]) return 1;   // the same walk over the edge records
         for (int g = 0; g < nlev; ++g) columns[(size_t)k * P + t0 + (size_t)(lv0 + g) * T] = v[g];
     }
     std::vector<uint2> entries(cap + 2u);
